@@ -136,6 +136,7 @@ _SIGNATURES = {
     "gpumpi_run_job": (ctypes.c_int, [_P, ctypes.POINTER(Job), _P, _P]),
     "gpumpi_job_heap_bytes": (ctypes.c_int64, [ctypes.POINTER(Job)]),
     "gpumpi_local_sort": (ctypes.c_int, [_P, ctypes.c_int64, _I32, _P, _P]),
+    "gpumpi_workspace_trim": (ctypes.c_int, []),
     "gpumpi_npb_is_run": (ctypes.c_int, [ctypes.c_char, _I32, ctypes.POINTER(ctypes.c_int64),
                                          ctypes.POINTER(ctypes.c_double)]),
     "gpumpi_gen_keys": (ctypes.c_int, [_P, _I32, ctypes.c_int64, ctypes.c_uint64, ctypes.c_uint32,
@@ -192,6 +193,13 @@ def local_sort(keys_ptr, n, key_bits, out_ptr, stream=0):
     rc = load_library().gpumpi_local_sort(keys_ptr, n, key_bits, out_ptr, stream or None)
     if rc != OK:
         raise GpumpiError(f"gpumpi_local_sort failed ({rc})")
+
+
+def workspace_trim():
+    """Give back the device memory that bucket_plan and local_sort keep between calls."""
+    rc = load_library().gpumpi_workspace_trim()
+    if rc != OK:
+        raise GpumpiError(f"gpumpi_workspace_trim failed ({rc})")
 
 
 def npb_is(cls, P):

@@ -1683,6 +1683,90 @@ int gpumpi_particles_phase_times(gpumpi_particle_plan* pl, int32_t enable, doubl
 
 }  // extern "C"
 
+// ==================================================================== workspaces
+// Device memory of one synchronous call, lent from a few idle blocks: hipMalloc and hipFree
+// (which waits for the whole device) cost more than a small call's kernels.  A block has one
+// user from the constructor to the destructor, and the call has waited for its stream
+// by then, so any thread, stream or device may take it next.  At most kIdleBlocks blocks and
+// kIdleBytes in all stay idle; gpumpi_workspace_trim gives them back, and so does an allocation
+// that fails.
+namespace {
+struct Workspace {
+    static constexpr size_t kIdleBlocks = 8, kIdleBytes = 64u << 20;
+    struct Block {
+        void* ptr;
+        size_t bytes;
+        int dev;
+    };
+    struct Pool {
+        std::mutex mu;
+        std::vector<Block> idle;
+        size_t bytes = 0;
+    };
+    static Pool& pool() {
+        static Pool* p = new Pool();   // outlives every static that may still call the library
+        return *p;
+    }
+    static int trim() {
+        std::vector<Block> gone;
+        {
+            std::lock_guard<std::mutex> g(pool().mu);
+            gone.swap(pool().idle);
+            pool().bytes = 0;
+        }
+        int rc = GPUMPI_OK;
+        for (const Block& b : gone)
+            if (hipFree(b.ptr) != hipSuccess) rc = GPUMPI_E_HIP;
+        return rc;
+    }
+
+    void* ptr = nullptr;
+    size_t bytes = 0;
+    int dev = -1;
+
+    explicit Workspace(size_t need) {
+        if (hipGetDevice(&dev) != hipSuccess) return;
+        bytes = 65536;
+        while (bytes < need) bytes *= 2;
+        if (need > kIdleBytes) bytes = need;     // never kept
+        {
+            std::lock_guard<std::mutex> g(pool().mu);
+            for (size_t i = 0; i < pool().idle.size(); i++) {
+                if (pool().idle[i].dev != dev || pool().idle[i].bytes != bytes) continue;
+                ptr = pool().idle[i].ptr;
+                pool().bytes -= bytes;
+                pool().idle.erase(pool().idle.begin() + (long)i);
+                return;
+            }
+        }
+        if (hipMalloc(&ptr, bytes) == hipSuccess) return;
+        (void)hipGetLastError();
+        ptr = nullptr;
+        trim();
+        if (hipMalloc(&ptr, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            ptr = nullptr;
+        }
+    }
+    ~Workspace() {
+        if (!ptr) return;
+        {
+            std::lock_guard<std::mutex> g(pool().mu);
+            if (bytes <= kIdleBytes - pool().bytes && pool().idle.size() < kIdleBlocks) {
+                pool().idle.push_back(Block{ptr, bytes, dev});
+                pool().bytes += bytes;
+                return;
+            }
+        }
+        hipFree(ptr);
+    }
+    Workspace(const Workspace&) = delete;
+    Workspace& operator=(const Workspace&) = delete;
+};
+}  // namespace
+
+extern "C" int gpumpi_workspace_trim(void) { return Workspace::trim(); }
+
 // ==================================================================== bucket-sort caller
 extern "C" {
 
@@ -1712,32 +1796,37 @@ int gpumpi_bucket_plan(const uint32_t* keys, int32_t P, int64_t n, int32_t key_b
     hipStream_t s = (hipStream_t)stream;
     const int nb = 1 << bucket_bits;
     const int shift = key_bits - bucket_bits;
-    uint32_t* hist = nullptr;
-    int64_t* totals = nullptr;
-    if (hipMalloc((void**)&hist, sizeof(uint32_t) * (size_t)P * nb) != hipSuccess) return GPUMPI_E_NOMEM;
-    if (hipMalloc((void**)&totals, sizeof(int64_t) * nb) != hipSuccess) {
-        hipFree(hist);
-        return GPUMPI_E_NOMEM;
-    }
+    // 16 keys per thread and tile; 4 where that leaves less than two workgroups per CU
+    const bool narrow = nb <= 1024;
+    const int64_t threads = narrow ? 1024 : 512;
+    const bool small = (int64_t)P * ((n + 16 * threads - 1) / (16 * threads)) < 512;
+    const int64_t tile_keys = (small ? 4 : 16) * threads;
+    const int64_t tiles64 = (n + tile_keys - 1) / tile_keys;
+    const int64_t grid64 = (int64_t)((P + 7) / 8 * 8) * tiles64;
+    if (grid64 > INT32_MAX) return GPUMPI_E_ARG;
+    const uint32_t tiles = (uint32_t)tiles64, grid = (uint32_t)grid64;
+    const bool cols = P > 64;   // up to 64 ranks the splitters' workgroup sums the columns itself
+    const size_t cnt_words = (size_t)P * tiles * nb, pre_words = (size_t)P * (nb + 1);
+    Workspace ws(sizeof(int64_t) * nb + sizeof(uint32_t) * (cnt_words + pre_words));
+    if (!ws.ptr) return GPUMPI_E_NOMEM;
+    int64_t* acc = (int64_t*)ws.ptr;
+    uint32_t* tile_cnt = (uint32_t*)(acc + nb);
+    uint32_t* prefix = tile_cnt + cnt_words;
+    hipLaunchKernelGGL(bucket_tile_hist_kernel, dim3(grid), dim3(kBucketThreads), sizeof(uint32_t) * nb, s, keys, P,
+                       n, shift, nb, (uint32_t)tile_keys, tiles, tile_cnt);
+    hipLaunchKernelGGL(bucket_rank_scan_kernel, dim3(P), dim3(kBucketThreads), 0, s, nb, tiles, tile_cnt, prefix);
+    if (cols)
+        hipLaunchKernelGGL(bucket_colsum_kernel, dim3((nb + kWave - 1) / kWave), dim3(kBucketThreads), 0, s, prefix, P,
+                           nb, acc);
+    hipLaunchKernelGGL(bucket_splitters_kernel, dim3(1), dim3(kBucketThreads), 0, s, cols ? acc : nullptr, prefix, P,
+                       nb, n, bucket_lo, bucket_hi);
+    auto scatter = narrow ? (small ? &bucket_scatter_kernel<1024, 4, 1024> : &bucket_scatter_kernel<1024, 16, 1024>)
+                          : (small ? &bucket_scatter_kernel<512, 4, 4096> : &bucket_scatter_kernel<512, 16, 4096>);
+    hipLaunchKernelGGL(scatter, dim3(grid), dim3((unsigned)threads), 0, s, keys, P, n, shift, nb, tiles, tile_cnt,
+                       prefix, bucket_lo, bucket_hi, key_buff1, send_counts, send_displs);
     int rc = GPUMPI_OK;
-    if (hipMemsetAsync(hist, 0, sizeof(uint32_t) * (size_t)P * nb, s) != hipSuccess) rc = GPUMPI_E_HIP;
-    int chunks = (int)((n + 256 * 64 - 1) / (256 * 64));
-    if (chunks > 64) chunks = 64;
-    hipLaunchKernelGGL(bucket_hist_kernel, dim3(chunks, P), dim3(256), sizeof(uint32_t) * nb, s,
-                       keys, n, shift, nb, hist);
-    hipLaunchKernelGGL(bucket_totals_kernel, dim3((nb + 255) / 256), dim3(256), 0, s, hist, P, nb,
-                       totals);
-    hipLaunchKernelGGL(bucket_splitters_kernel, dim3(1), dim3(64), 0, s, totals, P, nb, n,
-                       bucket_lo, bucket_hi);
-    hipLaunchKernelGGL(bucket_counts_kernel, dim3((P + 3) / 4), dim3(256), 0, s, hist, P, nb,
-                       bucket_lo, bucket_hi, send_counts, send_displs);
-    hipLaunchKernelGGL(bucket_scatter_kernel, dim3((P + 3) / 4), dim3(256),
-                       sizeof(uint32_t) * 4 * nb, s, keys, P, n, shift, nb, bucket_bits, hist,
-                       key_buff1);
     if (hipGetLastError() != hipSuccess) rc = GPUMPI_E_HIP;
     if (hipStreamSynchronize(s) != hipSuccess) rc = GPUMPI_E_HIP;
-    hipFree(hist);
-    hipFree(totals);
     return rc;
 }
 
@@ -2179,6 +2268,61 @@ int gpumpi_reduce_kernel_time(gpumpi_reduce_plan* pl, int32_t reps, void* stream
 }  // extern "C"
 
 // ==================================================================== local sort, NPB IS
+// Keys of at most kSortLowBits bits: one table, three launches.
+static int sort_short_keys(const uint32_t* keys, int64_t n, uint32_t bins, uint32_t* out, hipStream_t s) {
+    Workspace ws(sizeof(uint32_t) * bins);
+    if (!ws.ptr) return GPUMPI_E_NOMEM;
+    uint32_t* hist = (uint32_t*)ws.ptr;
+    // at most 512 workgroups add their counts to the table; a few of the expansion's tiles
+    // per workgroup, which scans the whole table
+    const int64_t step = 4 * kSortThreads;
+    const int64_t per = std::max<int64_t>(step, (n / 512 + step - 1) / step * step);
+    const int64_t outs = std::max<int64_t>(kSortTile, (n / 1024 + kSortTile - 1) / kSortTile * kSortTile);
+    hipLaunchKernelGGL(sort_zero_kernel, dim3((bins + kSortThreads - 1) / kSortThreads), dim3(kSortThreads), 0, s, hist,
+                       bins);
+    hipLaunchKernelGGL(sort_count_kernel, dim3((unsigned)((n + per - 1) / per)), dim3(kSortThreads), 0, s, keys, n, per,
+                       bins, hist);
+    hipLaunchKernelGGL(sort_expand_kernel, dim3((unsigned)((n + outs - 1) / outs)), dim3(kSortThreads), 0, s, hist, bins,
+                       n, outs, out);
+    const bool ok = hipGetLastError() == hipSuccess;
+    return hipStreamSynchronize(s) == hipSuccess && ok ? GPUMPI_OK : GPUMPI_E_HIP;
+}
+
+// Longer keys, split by their top bits into `parts` parts first.
+static int sort_by_parts(const uint32_t* keys, int64_t n, uint32_t parts, uint32_t* out, hipStream_t s) {
+    // a part is cut into chunks where one workgroup would hold up the others: about 512
+    // chunks of all keys, each worth the 2^14 counters it adds to the part's table
+    const int64_t chunk = std::min<int64_t>(262144, std::max<int64_t>(kSortTile, (n / 512 + kSortTile - 1) / kSortTile * kSortTile));
+    const int64_t most = 2 * chunk;
+    const uint32_t ntables = (uint32_t)std::min<int64_t>(parts, n / most);
+    const size_t words = (size_t)parts * 5 + 2;
+    Workspace ws(sizeof(uint32_t) * (words + (size_t)ntables * kSortBins));
+    if (!ws.ptr) return GPUMPI_E_NOMEM;
+    SortParts sp{};
+    sp.count = (uint32_t*)ws.ptr;
+    sp.first = sp.count + parts;
+    sp.moved = sp.first + parts + 1;
+    sp.item = sp.moved + parts;
+    sp.table = (int32_t*)(sp.item + parts + 1);
+    sp.tables = sp.count + words;
+    const int64_t step = 4 * kSortThreads;
+    const int64_t per = std::max<int64_t>(step, (n / 2048 + step - 1) / step * step);
+    const unsigned items = (unsigned)(parts + n / chunk);
+    hipLaunchKernelGGL(sort_zero_kernel, dim3(1), dim3(kSortThreads), 0, s, sp.count, parts);
+    hipLaunchKernelGGL(sort_top_hist_kernel, dim3((unsigned)((n + per - 1) / per)), dim3(kSortThreads), 0, s, keys, n,
+                       per, parts, sp.count);
+    hipLaunchKernelGGL(sort_top_scan_kernel, dim3(1), dim3(kSortThreads), 0, s, sp, parts, (uint32_t)most,
+                       (uint32_t)chunk);
+    hipLaunchKernelGGL(sort_split_kernel, dim3((unsigned)((n + kSortTile - 1) / kSortTile)), dim3(kSortThreads), 0, s,
+                       keys, n, sp, parts, ntables, out);
+    hipLaunchKernelGGL(sort_part_kernel, dim3(items), dim3(kSortThreads), 0, s, sp, parts, (uint32_t)chunk, out);
+    if (ntables)
+        hipLaunchKernelGGL(sort_part_expand_kernel, dim3(items), dim3(kSortThreads), 0, s, sp, parts, (uint32_t)chunk,
+                           out);
+    const bool ok = hipGetLastError() == hipSuccess;
+    return hipStreamSynchronize(s) == hipSuccess && ok ? GPUMPI_OK : GPUMPI_E_HIP;
+}
+
 extern "C" {
 
 int gpumpi_local_sort(const uint32_t* keys, int64_t n, int32_t key_bits, uint32_t* out,
@@ -2186,6 +2330,12 @@ int gpumpi_local_sort(const uint32_t* keys, int64_t n, int32_t key_bits, uint32_
     if (!keys || !out || n < 0 || n >= (1ll << 32) || key_bits < 1 || key_bits > 30)
         return GPUMPI_E_ARG;
     hipStream_t s = (hipStream_t)stream;
+    if (n == 0) return GPUMPI_OK;
+    const uintptr_t ka = (uintptr_t)keys, oa = (uintptr_t)out, len = sizeof(uint32_t) * (uintptr_t)n;
+    const bool overlap = ka < oa + len && oa < ka + len;
+    if (key_bits <= kSortLowBits) return sort_short_keys(keys, n, 1u << key_bits, out, s);
+    if (key_bits <= kSortLowBits + kSortTopBits && !overlap)
+        return sort_by_parts(keys, n, 1u << (key_bits - kSortLowBits), out, s);
     const uint32_t nbins = 1u << key_bits;
     const int nblk = (int)((nbins + 4095) / 4096);
     uint32_t *hist = nullptr, *prefix = nullptr, *big = nullptr, *nbig = nullptr;
@@ -2204,8 +2354,7 @@ int gpumpi_local_sort(const uint32_t* keys, int64_t n, int32_t key_bits, uint32_
         hipLaunchKernelGGL(scan_block_sums_kernel, dim3(nblk), dim3(1024), 0, s, hist, nbins, sums);
         hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, s, sums, nblk);
         hipLaunchKernelGGL(scan_apply_kernel, dim3(nblk), dim3(1024), 0, s, hist, nbins, sums, prefix);
-        hipLaunchKernelGGL(sort_expand_kernel, dim3(2048), dim3(256), 0, s, hist, prefix, nbins, out,
-                           big, nbig);
+        hipLaunchKernelGGL(sort_runs_kernel, dim3(2048), dim3(256), 0, s, hist, prefix, nbins, out, big, nbig);
         hipLaunchKernelGGL(sort_fill_runs_kernel, dim3(1024), dim3(256), 0, s, hist, prefix, big,
                            nbig, out);
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) rc = GPUMPI_E_HIP;

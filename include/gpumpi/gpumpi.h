@@ -336,6 +336,9 @@ int gpumpi_bucket_plan(const uint32_t* keys, int32_t P, int64_t n, int32_t key_b
  * at once (ranks own disjoint ascending key ranges; is.c:785-833 ranks by counting). */
 int gpumpi_local_sort(const uint32_t* keys, int64_t n, int32_t key_bits, uint32_t* out,
                       void* stream);
+/* Gives back the device memory that gpumpi_bucket_plan and gpumpi_local_sort keep idle between
+ * calls (at most 64 MiB). */
+int gpumpi_workspace_trim(void);
 /* NPB IS class cls ('S','W','A','B','C') on P ranks (power of two) through the batched
  * exchange: returns NPB's verification count in *passed (correct run: 5 * 10 + P,
  * is.c:1137-1138) and the summed exchange time of the 10 timed iterations. */
