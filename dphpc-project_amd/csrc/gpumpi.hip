@@ -915,8 +915,10 @@ static int a2av_configure(gpumpi_a2av_plan* pl, const gpumpi_a2av_tune& t) {
     if (t.pipeline < 0 || t.pipeline > 3) return GPUMPI_E_ARG;
     pl->tune.pipeline = t.pipeline;
     pl->dev.chunk_lines = (uint32_t)(kA2avCopyThreads * U * R);
+    pl->dev.min_lines = (uint32_t)(kA2avCopyThreads * U);
     a2av_size_grid(pl);
     pl->dev2.chunk_lines = pl->dev.chunk_lines;
+    pl->dev2.min_lines = pl->dev.min_lines;
     pl->dev2.straddle_blocks = pl->dev.straddle_blocks;
     return GPUMPI_OK;
 }
@@ -1056,9 +1058,9 @@ int gpumpi_a2av_plan_create(int32_t P, int32_t elem_bytes, void* const* sendbufs
     d.rcounts = recv_counts;
     d.rdispls = recv_displs;
     const uint64_t PP = (uint64_t)P * (uint64_t)P;
-    // per workspace: seg_end, seg_src [P*P], row_bytes [P], chunk_off [P+1], total bytes,
-    // plan-done counter (on its own 128-byte line)
-    const size_t ws = sizeof(uint64_t) * (2 * PP + P + (P + 1)) + 256;
+    // per workspace: seg_end, seg_src [P*P], row_bytes [P], chunk_off and short_off [P+1], total
+    // bytes and chunk lines, plan-done counter (on its own 128-byte line)
+    const size_t ws = sizeof(uint64_t) * (2 * PP + P + 2 * (P + 1)) + 256;
     char* w = nullptr;
     if (hipMalloc((void**)&w, 2 * ws) != hipSuccess) {
         delete pl;
@@ -1074,7 +1076,8 @@ int gpumpi_a2av_plan_create(int32_t P, int32_t elem_bytes, void* const* sendbufs
         x.seg_src = x.seg_end + PP;
         x.row_bytes = x.seg_src + PP;
         x.chunk_off = x.row_bytes + P;
-        x.total_bytes = (int64_t*)(x.chunk_off + P + 1);
+        x.short_off = x.chunk_off + P + 1;
+        x.total_bytes = (int64_t*)(x.short_off + P + 1);
         x.plan_done = (uint32_t*)(b + ws - 128);
     }
     for (int i = 0; i < 4; i++) hipEventCreate(&pl->ev[i]);
@@ -2054,7 +2057,7 @@ int64_t gpumpi_job_heap_bytes(const gpumpi_job* job) {
 // kernel reads it; nothing has to start at zero.
 constexpr int32_t kNoAllocMaxRanks = 512;
 constexpr size_t kNoAllocScratchBytes =
-    sizeof(uint64_t) * (2ull * kNoAllocMaxRanks * kNoAllocMaxRanks + 2ull * kNoAllocMaxRanks + 2) + 256;
+    sizeof(uint64_t) * (2ull * kNoAllocMaxRanks * kNoAllocMaxRanks + 3ull * kNoAllocMaxRanks + 2) + 256;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -2115,9 +2118,11 @@ int gpumpi_a2av_execute_noalloc(int32_t P, int32_t elem_bytes, void* const* send
     d.seg_src = d.seg_end + PP;
     d.row_bytes = d.seg_src + PP;
     d.chunk_off = d.row_bytes + P;
-    d.total_bytes = (int64_t*)(d.chunk_off + P + 1);
+    d.short_off = d.chunk_off + P + 1;
+    d.total_bytes = (int64_t*)(d.short_off + P + 1);
     d.plan_done = nullptr;
     d.chunk_lines = (uint32_t)(kA2avCopyThreads * 4 * 2);  // 4 lines per lane, 2 rounds
+    d.min_lines = (uint32_t)(kA2avCopyThreads * 4);
     d.straddle_blocks = 0;
     hipStream_t s = (hipStream_t)stream;
     void* kargs1[] = {(void*)&d};

@@ -29,9 +29,14 @@
 //         16-byte store -- or, in
 //         deferred mode (a tuning choice that pays when segments are short, as in skewed
 //         key distributions), left to one thread per segment run by the grid's first
-//         blocks, concurrently with the streaming blocks.  Lines at a row's ends, and
-//         dwords that are split or unaligned at the source, go byte by byte; bytes outside
-//         the row are never written.
+//         blocks, concurrently with the streaming blocks.  Dwords that are split or unaligned
+//         at the source go byte by byte; bytes outside the row are never written.  The lines
+//         at the ends of rows are a lane each in the first blocks.
+//         Rows of short segments, of elements that are not whole dwords, and small rows take
+//         a loop of their own (a2av_copy_short), in which each lane finds its line's segments.
+//         Measured (execute, us, before -> with it): 16 ranks x 3 KiB 24.0 -> 12.9; 200 ranks,
+//         48 MiB of bytes, segments of 157 B to 50 KiB 403 -> 39; 512 ranks, 64-byte segments,
+//         16 MiB 95 -> 35.
 //
 // Why not one persistent kernel with a grid barrier: on gfx950 an agent-scope release or
 // acquire writes back or invalidates the XCD's L2 (buffer_wbl2 / buffer_inv sc1); a grid
@@ -50,10 +55,29 @@ namespace gpumpi {
 constexpr int kA2avWindow = 64;
 constexpr int kA2avCopyThreads = 256;
 
+// Short rows are copied line by line (a2av_copy_short): every lane finds its own line's
+// segments.  Their chunks are smaller, so that more workgroups share them.  A row is short
+// when its non-empty segments average less than kA2avShortBytes (kA2avShortOdd if the elements
+// are not whole dwords, which the other loop assembles byte by byte at every boundary), or when
+// it is too small to be a stream at all.  Where the lines lie, measured (short / long loop, us):
+// 256 ranks of dwords, segments of 256 B 24.9 / 38.7, 512 B 33.6 / 32.3, 1 KiB 49 / 38; of
+// bytes, 4 KiB 147 / 257, 16 KiB 516 / 706, 64 KiB (32 ranks) 39 / 37; 4 ranks x 4 KiB rows
+// 13.3 / 15.4, 8 KiB 12.6 / 13.0, 16 KiB 13.6 / 12.8.
+constexpr uint64_t kA2avShortRow = 1ull << 63;
+constexpr uint64_t kA2avShortBytes = 448;
+constexpr uint64_t kA2avShortOdd = 32768;
+constexpr uint64_t kA2avSmallRow = 8192;
+// Lines per chunk of a short row: 16 KiB, up to 64 KiB in steps that give twice kA2avChunks of
+// them (finding a chunk's row and segments takes about as long as copying 16 KiB).
+constexpr uint64_t kA2avShortLines = 1024, kA2avShortMost = 4096;
+constexpr int kA2avShortWindow = 512;
+constexpr uint64_t kA2avChunks = 2048;    // chunks that keep the chip busy
+
 struct A2avDev {
     int32_t P;
     int32_t elem;
-    uint32_t chunk_lines;   // destination lines per chunk = kA2avCopyThreads * U
+    uint32_t chunk_lines;   // destination lines per chunk at most: kA2avCopyThreads * U * rounds
+    uint32_t min_lines;     // and at least: kA2avCopyThreads * U
     int32_t straddle_blocks;  // deferred mode: leading copy blocks running the straddle threads
     char* const* sendbufs;
     const int32_t* scounts;
@@ -63,9 +87,10 @@ struct A2avDev {
     int32_t* rdispls;
     uint64_t* seg_end;      // [P*P] end byte offset of segment (d, s) within row d
     uint64_t* seg_src;      // [P*P] address of the first source byte of segment (d, s)
-    uint64_t* row_bytes;    // [P]
-    uint64_t* chunk_off;    // [P+1] exclusive prefix of chunks per row; [P] = total chunks
-    int64_t* total_bytes;   // [1]
+    uint64_t* row_bytes;    // [P], with kA2avShortRow set in rows of short segments
+    uint64_t* chunk_off;    // [P+1] exclusive prefix of chunks per long row; [P] = all of them
+    uint64_t* short_off;    // [P+1] the same for the short rows
+    int64_t* total_bytes;   // [0] payload; [1] lines per chunk of the long rows, [2] of the short
     uint32_t* plan_done;    // [1] plan workgroups finished (fused plan; reset by the last one)
 };
 
@@ -112,7 +137,8 @@ __device__ __forceinline__ void a2av_plan_row(const A2avDev& p, int64_t d, int64
     const int se = sb + Q < P ? sb + Q : P;
     int64_t c[4], sd[4];
     const char* sbuf[4];
-    int64_t part = 0;
+    int64_t part = 0;        // elements, and non-empty segments from bit 44 on
+    constexpr int kSegShift = 44;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int s = sb + q * kWave + l;
@@ -120,19 +146,22 @@ __device__ __forceinline__ void a2av_plan_row(const A2avDev& p, int64_t d, int64
         c[q] = valid ? p.scounts[(int64_t)s * P + d] : 0;
         sd[q] = valid ? p.sdispls[(int64_t)s * P + d] : 0;
         sbuf[q] = valid ? p.sendbufs[s] : nullptr;
-        part += c[q];
+        part += c[q] + (c[q] > 0 ? 1ll << kSegShift : 0);
     }
     for (int s0 = sb + 4 * kWave; s0 < se; s0 += kWave) {
         const int s = s0 + l;
-        part += s < se ? p.scounts[(int64_t)s * P + d] : 0;
+        const int64_t x = s < se ? p.scounts[(int64_t)s * P + d] : 0;
+        part += x + (x > 0 ? 1ll << kSegShift : 0);
     }
     part = wave_sum(part);
     if (l == 0) s_tot[w] = part;
     __syncthreads();
-    int64_t carry = 0, row = 0;
+    int64_t carry = 0, row = 0, nonempty = 0;
     for (int k = 0; k < 4; k++) {
-        carry += k < w ? s_tot[k] : 0;
-        row += s_tot[k];
+        const int64_t x = s_tot[k] & ((1ll << kSegShift) - 1);
+        carry += k < w ? x : 0;
+        row += x;
+        nonempty += s_tot[k] >> kSegShift;
     }
     for (int s0 = sb; s0 < se; s0 += kWave) {
         const int q = (s0 - sb) / kWave;
@@ -161,7 +190,11 @@ __device__ __forceinline__ void a2av_plan_row(const A2avDev& p, int64_t d, int64
         }
     }
     if (threadIdx.x == 0) {
-        const uint64_t rb = (uint64_t)row * (uint64_t)p.elem;
+        uint64_t rb = (uint64_t)row * (uint64_t)p.elem;
+        // (deferred mode has its own way with short segments)
+        if (p.straddle_blocks == 0 &&
+            (rb < kA2avSmallRow || rb < (uint64_t)nonempty * (p.elem & 3 ? kA2avShortOdd : kA2avShortBytes)))
+            rb |= kA2avShortRow;
         if constexpr (COHERENT) st_relaxed(&p.row_bytes[d], rb);
         else p.row_bytes[d] = rb;
     }
@@ -180,37 +213,54 @@ __device__ __forceinline__ void a2av_scan_rows(const A2avDev& p, uint64_t* part,
     constexpr int NW = NT / kWave;
     const int P = p.P;
     const int w = threadIdx.x >> 6;
-    const uint64_t C = p.chunk_lines;
-    uint64_t carry = 0;
+    auto row_word = [&](int d) { return COHERENT ? ld_relaxed(&p.row_bytes[d]) : p.row_bytes[d]; };
     int64_t bytes = 0;
     for (int base = 0; base < P; base += NT) {
         const int d = base + (int)threadIdx.x;
+        bytes += d < P ? (int64_t)(row_word(d) & ~kA2avShortRow) : 0;
+    }
+    bytes = wave_sum(bytes);
+    if (lane() == 0) bpart[w] = bytes;
+    __syncthreads();
+    bytes = 0;
+    for (int k = 0; k < NW; k++) bytes += bpart[k];
+    // smaller chunks while the payload does not give kA2avChunks of them
+    uint64_t C = p.chunk_lines;
+    while (C > p.min_lines && (uint64_t)bytes / 16 < C * kA2avChunks) C >>= 1;
+    uint64_t S = kA2avShortMost;
+    while (S > kA2avShortLines && (uint64_t)bytes / 16 < S * 2 * kA2avChunks) S >>= 1;
+    uint64_t carry = 0;      // chunks of long rows, and of short rows from bit 32 on
+    for (int base = 0; base < P; base += NT) {
+        const int d = base + (int)threadIdx.x;
         uint64_t ch = 0;
-        int64_t nb = 0;
         if (d < P) {
-            nb = COHERENT ? (int64_t)ld_relaxed(&p.row_bytes[d]) : (int64_t)p.row_bytes[d];
+            const uint64_t word = row_word(d), nb = word & ~kA2avShortRow;
             const uint64_t rb = (uint64_t)(uintptr_t)p.recvbufs[d];
-            const uint64_t lines = nb ? ((rb + (uint64_t)nb + 15) >> 4) - ((rb >> 7) << 3) : 0;
-            ch = (lines + C - 1) / C;
+            const uint64_t lines = nb ? ((rb + nb + 15) >> 4) - ((rb >> 7) << 3) : 0;
+            ch = word & kA2avShortRow ? ((lines + S - 1) / S) << 32 : (lines + C - 1) / C;
         }
         const uint64_t inc = (uint64_t)wave_incl_scan((int64_t)ch);
-        const int64_t bsum = wave_sum(nb);
         if (lane() == 63) part[w] = inc;
-        if (lane() == 0) bpart[w] = bsum;
         __syncthreads();
         uint64_t before = 0, total = 0;
         for (int k = 0; k < NW; k++) {
             if (k < w) before += part[k];
             total += part[k];
-            bytes += (threadIdx.x == 0) ? bpart[k] : 0;
         }
-        if (d < P) p.chunk_off[d] = carry + before + inc - ch;
+        if (d < P) {
+            const uint64_t off = carry + before + inc - ch;
+            p.chunk_off[d] = (uint32_t)off;
+            p.short_off[d] = off >> 32;
+        }
         carry += total;
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        p.chunk_off[P] = carry;
-        *p.total_bytes = bytes;
+        p.chunk_off[P] = (uint32_t)carry;
+        p.short_off[P] = carry >> 32;
+        p.total_bytes[0] = bytes;
+        p.total_bytes[1] = (int64_t)C;
+        p.total_bytes[2] = (int64_t)S;
     }
 }
 
@@ -277,7 +327,7 @@ __device__ void a2av_straddle_line(const A2avDev& p, uint64_t gid) {
     const uint64_t src0 = p.seg_src[d * P + s];
     const uint64_t src1 = p.seg_src[d * P + s1];
     const uint64_t rbase = (uint64_t)(uintptr_t)p.recvbufs[d];
-    const int64_t rbytes = (int64_t)p.row_bytes[d];
+    const int64_t rbytes = (int64_t)(p.row_bytes[d] & ~kA2avShortRow);
     const int64_t st = s > 0 ? prev : 0;
     if (en <= st) return;  // empty
     const uint64_t le = rbase + (uint64_t)en;  // one past the segment's last byte
@@ -411,17 +461,109 @@ __device__ __forceinline__ A2avSegView a2av_seg_at(const A2avDev& p, int64_t d, 
     return a2av_seg_global(p, d, rbase, q);
 }
 
-// A destination line that straddles segments or the row's ends: assembled per dword
-// (per byte where a dword is split or its source unaligned); only row bytes are written.
-// In deferred mode the lines inside the row are the straddle threads'.
+// 16 bytes from byte `at` (0..16) of the 32 bytes a, b.
+__device__ __forceinline__ u32x4 bytes_from(u32x4 a, u32x4 b, uint32_t at) {
+    const bool h16 = at & 16, h8 = at & 8, h4 = at & 4;
+    // (scalars: an array would be indexed in scratch memory)
+    uint32_t x0 = h16 ? b.x : a.x, x1 = h16 ? b.y : a.y, x2 = h16 ? b.z : a.z, x3 = h16 ? b.w : a.w;
+    uint32_t x4 = b.x, x5 = b.y, x6 = b.z;       // (past byte 16 nothing follows)
+    x0 = h8 ? x2 : x0;
+    x1 = h8 ? x3 : x1;
+    x2 = h8 ? x4 : x2;
+    x3 = h8 ? x5 : x3;
+    x4 = h8 ? x6 : x4;
+    x5 = h8 ? b.w : x5;
+    x0 = h4 ? x1 : x0;
+    x1 = h4 ? x2 : x1;
+    x2 = h4 ? x3 : x2;
+    x3 = h4 ? x4 : x3;
+    x4 = h4 ? x5 : x4;
+    return u32x4{(uint32_t)__builtin_amdgcn_alignbyte(x1, x0, at), (uint32_t)__builtin_amdgcn_alignbyte(x2, x1, at),
+                 (uint32_t)__builtin_amdgcn_alignbyte(x3, x2, at), (uint32_t)__builtin_amdgcn_alignbyte(x4, x3, at)};
+}
+
+// Bytes [0, n) at address a, n < 16, in the low bytes; reads nothing else.
+__device__ __forceinline__ u32x4 load_bytes(uint64_t a, uint32_t n) {
+    typedef uint64_t u64_a1 __attribute__((aligned(1)));
+    typedef uint32_t u32_a1 __attribute__((aligned(1)));
+    typedef uint16_t u16_a1 __attribute__((aligned(1)));
+    uint64_t lo = 0, r = 0;
+    uint32_t f = 0, g = 0;
+    if (n & 8) {
+        lo = *(const GPUMPI_GLOBAL u64_a1*)(uintptr_t)a;
+        f = 8;
+    }
+    if (n & 4) {
+        r = *(const GPUMPI_GLOBAL u32_a1*)(uintptr_t)(a + f);
+        g = 4;
+    }
+    if (n & 2) {
+        r |= (uint64_t)*(const GPUMPI_GLOBAL u16_a1*)(uintptr_t)(a + f + g) << (8 * g);
+        g += 2;
+    }
+    if (n & 1) r |= (uint64_t)*(const GPUMPI_GLOBAL uint8_t*)(uintptr_t)(a + f + g) << (8 * g);
+    if (!(n & 8)) { lo = r; r = 0; }
+    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)r, (uint32_t)(r >> 32)};
+}
+
+// The destination line `line` of a row, from however many segments it holds: at(q) is the
+// segment holding row byte q.  Each piece is one 16-byte load from inside its segment, moved to
+// its bytes (a segment of less than 16 bytes: up to four smaller loads); only row bytes are
+// read and written.  A byte at a time -- a search, a load and a store for each of 16 -- such lines took
+// most of a copy of short unaligned segments.
+template <class F>
+__device__ __forceinline__ void a2av_assemble_line(uint64_t rbase, int64_t rbytes, uint64_t line, F at) {
+    const uint64_t la = line << 4;
+    const int64_t off = (int64_t)la - (int64_t)rbase;
+    const int b0 = off >= 0 ? 0 : off <= -16 ? 16 : (int)-off;
+    const int b1 = rbytes - off >= 16 ? 16 : (int)(rbytes - off);
+    if (b0 >= b1) return;
+    uint32_t acc[4] = {0, 0, 0, 0};
+    for (int pos = b0; pos < b1;) {
+        const A2avSegView sg = at(off + pos);
+        const int64_t end = sg.en - off, start = sg.st - off;      // in line bytes
+        const int e = end < b1 ? (int)end : b1;
+        const uint64_t src = la + sg.D;                            // of line byte 0
+        const u32x4 none{0u, 0u, 0u, 0u};
+        u32x4 y;
+        if (end - start >= 16) {
+            int64_t f = start > 0 ? start : 0;
+            if (f > end - 16) f = end - 16;                        // -15 .. 15
+            const u32x4 x = gload16(src + (uint64_t)f);
+            y = bytes_from(f >= 0 ? none : x, f >= 0 ? x : none, (uint32_t)(f >= 0 ? 16 - f : -f));
+        } else {
+            y = bytes_from(none, load_bytes(src + (uint64_t)pos, (uint32_t)(e - pos)), 16u - (uint32_t)pos);
+        }
+        const uint32_t w[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int a = pos - 4 * i, b = e - 4 * i;
+            const uint64_t upto = (1ull << (8 * (b < 0 ? 0 : b > 4 ? 4 : b))) - 1;
+            const uint64_t skip = (1ull << (8 * (a < 0 ? 0 : a > 4 ? 4 : a))) - 1;
+            acc[i] |= w[i] & (uint32_t)(upto & ~skip);
+        }
+        pos = e;
+    }
+    if (b0 == 0 && b1 == 16) {
+        *(GPUMPI_GLOBAL u32x4*)(uintptr_t)la = u32x4{acc[0], acc[1], acc[2], acc[3]};
+        return;
+    }
+    for (int b = b0; b < b1; b++) {
+        const uint32_t x = b < 4 ? acc[0] : b < 8 ? acc[1] : b < 12 ? acc[2] : acc[3];
+        *(GPUMPI_GLOBAL uint8_t*)(uintptr_t)(la + b) = (uint8_t)(x >> (8 * (b & 3)));
+    }
+}
+
+// A destination line that straddles segments (deferred mode, whose straddle threads have
+// those: the row's ends): assembled per dword (per byte where a dword is split or its source
+// unaligned); only row bytes are written.
 template <bool DEFER>
 __device__ void a2av_boundary_line(const A2avDev& p, int64_t d, uint64_t rbase, int64_t rbytes,
                                    const A2avWin& w, uint64_t line) {
     const uint64_t la = line << 4;
     const int64_t off = (int64_t)la - (int64_t)rbase;
-    if constexpr (DEFER) {
-        if (off >= 0 && off + 16 <= rbytes) return;
-    }
+    // deferred mode: only the lines at the row's ends are left; otherwise only those inside it
+    if (DEFER == (off >= 0 && off + 16 <= rbytes)) return;
     uint32_t v[4] = {0, 0, 0, 0};
     int mask = 0;
     for (int i = 0; i < 4; i++) {
@@ -451,6 +593,146 @@ __device__ void a2av_boundary_line(const A2avDev& p, int64_t d, uint64_t rbase, 
     }
 }
 
+// The first (which = 0) or last line of long row d, if it holds bytes of the row and others.
+// (Left to the copy loop, whose lane assembles it byte by byte, such a line holds up the
+// workgroup that ends its row by some 20 us.)
+__device__ __forceinline__ void a2av_row_end(const A2avDev& p, int64_t d, int which) {
+    const uint64_t word = p.row_bytes[d];
+    if (word == 0 || (word & kA2avShortRow)) return;
+    const uint64_t rbase = (uint64_t)(uintptr_t)p.recvbufs[d], rend = rbase + word;
+    if (((which ? rend : rbase) & 15) == 0) return;
+    const uint64_t first = rbase >> 4, last = rend >> 4;
+    if (which && first == last && (rbase & 15)) return;     // one line: the first
+    a2av_assemble_line(rbase, (int64_t)word, which ? last : first,
+                       [&](int64_t q) { return a2av_seg_global(p, d, rbase, q); });
+}
+
+// Lines [pos, line1) of a row of short segments, by the whole workgroup.  Windows of up
+// to 512 segments in LDS (offsets relative to the window's first row byte `o`); each lane finds the
+// segment of its line by bisection, four lines at a time, so that the searches' LDS reads and
+// the lines' loads overlap.  A line across one boundary takes the 16 bytes up to the
+// boundary and the 16 from it, and a funnel shift; other lines are assembled piece by piece.
+// A wave-uniform cursor over the segments (the loop for long segments) gains nothing when
+// every slice of 64 lines crosses several.
+template <bool NT>
+__device__ __forceinline__ void a2av_copy_short(const A2avDev& p, int64_t d, uint64_t rbase, int64_t rbytes,
+                                                uint64_t pos, uint64_t line1, int32_t* sE, uint64_t* sD,
+                                                int64_t* meta) {
+    constexpr int U = 2;
+    const int P = p.P;
+    const int tid = threadIdx.x;
+    const uint64_t* se = p.seg_end + d * P;
+    const uint64_t* src = p.seg_src + d * P;
+    // twice the segments that a chunk of the row holds on average
+    const uint64_t avg = 2 * 16 * (line1 - pos) * (uint64_t)P / (uint64_t)rbytes + 16;
+    const int most = avg < kA2avShortWindow ? (int)avg : kA2avShortWindow;
+    while (pos < line1) {
+        const int64_t o0 = (int64_t)(pos << 4) - (int64_t)rbase;
+        const int64_t o = o0 < 0 ? 0 : o0;
+        if (tid < kWave) {
+            int64_t s0 = 0;
+            if ((int64_t)se[0] <= o) s0 = wave_search_le(se, P, (uint64_t)o) + 1;
+            if (tid == 0) meta[5] = s0;
+        }
+        __syncthreads();
+        const int s0 = (int)bcast(meta[5]);
+        const int n = P - s0 < most ? P - s0 : most;
+        for (int k = tid; k < n; k += kA2avCopyThreads) {
+            const int s = s0 + k;
+            const int64_t en = (int64_t)se[s], st = s > 0 ? (int64_t)se[s - 1] : 0;
+            sE[k] = (int32_t)(en - o < INT32_MAX ? en - o : INT32_MAX);
+            sD[k] = src[s] - (rbase + (uint64_t)st);
+            if (k == 0) meta[6] = st - o > INT32_MIN / 2 ? st - o : INT32_MIN / 2;
+            if (k == n - 1) meta[7] = en;
+        }
+        __syncthreads();
+        const int32_t start0 = (int32_t)bcast(meta[6]);
+        const int64_t cover = bcast(meta[7]);
+        // lines inside the window's coverage; to the row's end when the window reaches it
+        uint64_t pend = s0 + n >= P ? line1 : (rbase + (uint64_t)cover) >> 4;
+        if (pend > line1) pend = line1;
+        if (pend <= pos) {     // more segments in one line than the window holds
+            if (tid == 0)
+                a2av_assemble_line(rbase, rbytes, pos, [&](int64_t q) { return a2av_seg_global(p, d, rbase, q); });
+            pos++;
+            __syncthreads();
+            continue;
+        }
+        const int top = n > 1 ? 1 << (31 - __builtin_clz(n - 1)) : 0;
+        auto find = [&](int32_t q) {       // first entry that ends past q
+            int k = 0;
+            for (int b = top; b > 0; b >>= 1)
+                if (k + b <= n - 1 && sE[k + b - 1] <= q) k += b;
+            return k;
+        };
+        for (uint64_t base = pos; base < pend; base += (uint64_t)kA2avCopyThreads * U) {
+            int32_t q[U];      // window offset of the line's first row byte
+            int k[U], kind[U]; // 0 none, 1 one segment, 2 two segments, 3 assemble
+            uint32_t cut[U];
+            u32x4 v[U], w[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint64_t line = base + (uint64_t)u * kA2avCopyThreads + tid;
+                const int64_t off = (int64_t)(line << 4) - (int64_t)rbase;
+                kind[u] = line < pend && off > -16 ? off < 0 || off + 16 > rbytes ? 3 : 1 : 0;
+                q[u] = kind[u] ? (int32_t)(off - o) : 0;
+                if (q[u] < 0) q[u] = 0;
+                k[u] = 0;
+            }
+            for (int b = top; b > 0; b >>= 1) {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int at = k[u] + b <= n - 1 ? k[u] + b : 0;
+                    if (at && sE[at - 1] <= q[u]) k[u] = at;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (kind[u] != 1) continue;
+                const uint64_t la = (base + (uint64_t)u * kA2avCopyThreads + tid) << 4;
+                const int32_t e = sE[k[u]];
+                if (e - q[u] >= 16) {
+                    v[u] = gload16(la + sD[k[u]]);
+                    continue;
+                }
+                // the next non-empty segment; the one after the line's last byte at most
+                int k2 = k[u] + 1;
+                while (k2 < n - 1 && sE[k2] <= e) k2++;
+                const int32_t st = k[u] > 0 ? sE[k[u] - 1] : start0;
+                if (k2 < n && sE[k2] - e >= 16 && e - st >= 16) {
+                    const uint32_t a = (uint32_t)(e - q[u]);       // bytes from the first segment
+                    v[u] = gload16(la + a - 16 + sD[k[u]]);
+                    w[u] = gload16(la + a + sD[k2]);
+                    cut[u] = 16 - a;
+                    kind[u] = 2;
+                } else {
+                    kind[u] = 3;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint64_t la = (base + (uint64_t)u * kA2avCopyThreads + tid) << 4;
+                if (kind[u] == 2) v[u] = bytes_from(v[u], w[u], cut[u]);
+                if (kind[u] == 1 || kind[u] == 2) gstore16<NT>(la, v[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (kind[u] != 3) continue;
+                a2av_assemble_line(rbase, rbytes, base + (uint64_t)u * kA2avCopyThreads + tid, [&](int64_t x) {
+                    const int j = find((int32_t)(x - o));
+                    A2avSegView g;
+                    g.st = o + (j > 0 ? sE[j - 1] : start0);
+                    g.en = o + sE[j];
+                    g.D = sD[j];
+                    return g;
+                });
+            }
+        }
+        __syncthreads();
+        pos = pend;
+    }
+}
+
 // FUSE: the first pn.P workgroups plan the next step into pn (a2av_plan_fused); the copy
 // workgroups follow them.
 template <int U, bool NT, bool DEFER, bool FUSE>
@@ -459,10 +741,11 @@ __global__ void __launch_bounds__(kA2avCopyThreads) a2av_copy_kernel(A2avDev p, 
     __shared__ int64_t s_en[kA2avWindow];
     __shared__ uint64_t s_D[kA2avWindow];
     __shared__ int64_t s_meta[10];
+    __shared__ int32_t s_E[DEFER ? 1 : kA2avShortWindow];
+    __shared__ uint64_t s_DW[DEFER ? 1 : kA2avShortWindow];
     const int P = p.P;
     const int tid = threadIdx.x;
     const int l = lane();
-    const uint64_t C = p.chunk_lines;
     uint32_t bid = blockIdx.x, nblk = gridDim.x;
     if constexpr (FUSE) {
         if (bid < (uint32_t)pn.P) {  // block-uniform
@@ -483,8 +766,15 @@ __global__ void __launch_bounds__(kA2avCopyThreads) a2av_copy_kernel(A2avDev p, 
             return;
         }
     }
+    // the partial lines at the ends of the long rows: a lane each, in the first blocks
+    if constexpr (!DEFER) {
+        for (uint64_t g = (uint64_t)bid * kA2avCopyThreads + tid; g < 2 * (uint64_t)P; g += (uint64_t)nblk * kA2avCopyThreads)
+            a2av_row_end(p, (int64_t)(g >> 1), (int)(g & 1));
+    }
     const uint64_t total = p.chunk_off[P];
-    for (uint64_t ch = bid - sb; ch < total; ch += nblk - sb) {
+    const uint64_t C = (uint64_t)p.total_bytes[1];
+    uint64_t ch = bid - sb;
+    for (; ch < total; ch += nblk - sb) {
         // ---- the chunk's row and line range
         if (tid < kWave) {
             const int64_t d = wave_search_le(p.chunk_off, P, ch);
@@ -678,6 +968,29 @@ __global__ void __launch_bounds__(kA2avCopyThreads) a2av_copy_kernel(A2avDev p, 
             }
             __syncthreads();
             pos = pend;
+        }
+    }
+    // the short rows' chunks follow the long rows' in a loop of their own: in one loop, the
+    // registers of the loads above stay live through this path (115 instead of 87)
+    if constexpr (!DEFER) {
+        const uint64_t shorts = p.short_off[P], S = (uint64_t)p.total_bytes[2];
+        for (; ch - total < shorts; ch += nblk) {
+            if (tid < kWave) {
+                const int64_t d = wave_search_le(p.short_off, P, ch - total);
+                if (l == 0) {
+                    s_meta[0] = d;
+                    s_meta[1] = (int64_t)(ch - total - p.short_off[d]);
+                }
+            }
+            __syncthreads();
+            const int64_t d = bcast(s_meta[0]);
+            const uint64_t c = (uint64_t)bcast(s_meta[1]);
+            const uint64_t rbase = (uint64_t)(uintptr_t)p.recvbufs[d];
+            const int64_t rbytes = (int64_t)(p.row_bytes[d] & ~kA2avShortRow);
+            const uint64_t lend = (rbase + (uint64_t)rbytes + 15) >> 4;
+            const uint64_t line0 = ((rbase >> 7) << 3) + c * S;
+            const uint64_t line1 = line0 + S < lend ? line0 + S : lend;
+            a2av_copy_short<NT>(p, d, rbase, rbytes, line0, line1, s_E, s_DW, s_meta);
         }
     }
 }
