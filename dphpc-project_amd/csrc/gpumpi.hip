@@ -2143,13 +2143,33 @@ struct gpumpi_reduce_plan {
     ReduceDev dev{};
     const void* kernel = nullptr;
     int grid = 0;
+    int32_t log_cols = 0;    // staged kernel: columns per tile
     std::vector<A2avGraph> graphs;
 };
 
 static int reduce_launch(gpumpi_reduce_plan* pl, hipStream_t s) {
-    void* kargs[] = {(void*)&pl->dev};
+    void* kargs[] = {(void*)&pl->dev, (void*)&pl->log_cols};   // (the other kernels take the first)
     return hipLaunchKernel(pl->kernel, dim3(pl->grid), dim3(kReduceThreads), kargs, 0, s) == hipSuccess
                ? GPUMPI_OK : GPUMPI_E_HIP;
+}
+
+// Whether buffers of `bytes` take the staged kernel: those with too few tiles for the kernels
+// that fold from HBM.  Measured (Allreduce of doubles, from HBM / staged, us): 1024 ranks x 4
+// KiB 165 / 24, 64 KiB 169 / 42, 256 KiB 168 / 129, 768 KiB 338 / 410; 512 ranks x 256 KiB
+// 85 / 45, 384 KiB 89 / 104; 32 ranks x 4 KiB 6.8 / 3.2, 512 KiB 9.8 / 7.7, 768 KiB 11 / 12.
+// The split fold of whole numbers (4 ranks and more) is passed up to 128 KiB: int32, 1024
+// ranks x 64 KiB 54 / 39, 128 KiB 59 / 52, 256 KiB 95 / 129.
+static bool reduce_is_staged(int32_t P, uint64_t bytes, bool split) {
+    if (split) return bytes <= (128u << 10);
+    return bytes <= (P <= 64 ? 512u << 10 : 256u << 10);
+}
+
+// 16-byte columns per tile of the staged kernel (log2): 4 workgroups per CU, but 128-byte
+// tiles and more while those give 2 (1024 ranks x 64 KiB: 128-byte tiles 42 us, 64-byte 45).
+static int reduce_staged_cols(uint64_t cols, uint64_t cus) {
+    int k = 6;
+    while (k > 3 && cols >> k < 4 * cus) k--;
+    return k == 3 && cols >> 3 < 2 * cus ? 2 : k;
 }
 
 extern "C" {
@@ -2167,7 +2187,8 @@ int gpumpi_reduce_plan_create(int32_t P, int64_t count, int32_t datatype, int32_
     const bool wide = bytes / (1024ull * kReduceWideU) >= 4ull * (uint64_t)cus;
     // integer pairs below the wide shape fold with the ranks split over a workgroup's waves
     const void* ks = es > 0 && !wide && P >= kReduceSplitWaves ? batched_reduce_split_lookup(datatype, op) : nullptr;
-    const void* k = ks ? ks : es > 0 ? batched_reduce_kernel_lookup(datatype, op, wide) : nullptr;
+    const void* kst = es > 0 && reduce_is_staged(P, bytes, ks != nullptr) ? batched_reduce_staged_lookup(datatype, op) : nullptr;
+    const void* k = kst ? kst : ks ? ks : es > 0 ? batched_reduce_kernel_lookup(datatype, op, wide) : nullptr;
     if (!k) {
         g_host_error = "batched reduction: the pair (datatype " + std::to_string(datatype) +
                        ", operator " + std::to_string(op) + ") is not on the batched path "
@@ -2184,9 +2205,16 @@ int gpumpi_reduce_plan_create(int32_t P, int64_t count, int32_t datatype, int32_
     pl->dev.nt = written >= (64ull << 20) ? 1 : 0;  // outputs larger than the L2s stream past them
     pl->dev.sendbufs = (const char*)sendbufs;
     pl->dev.recvbufs = (const char*)recvbufs;
-    uint64_t g = ks ? batched_reduce_split_grid(bytes)
+    uint64_t g = ks && !kst ? batched_reduce_split_grid(bytes)
                     : batched_reduce_grid(bytes, wide ? kReduceWideU : kReduceNarrowU);
+    if (kst) {
+        const uint64_t cols = (bytes + 15) / 16;
+        pl->log_cols = reduce_staged_cols(cols, (uint64_t)cus);
+        g = (cols + (1ull << pl->log_cols) - 1) >> pl->log_cols;
+    }
     if (g > (1u << 20)) g = 1u << 20;  // the waves stride over the rest
+    if (g < 1) g = 1;
+    if (!kst && bytes % 16) g++;       // the partial last column's workgroup
     pl->grid = (int)g;
     *out = pl;
     return GPUMPI_OK;

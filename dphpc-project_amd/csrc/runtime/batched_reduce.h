@@ -9,9 +9,9 @@
 //
 // The reference runs this as P-1 point-to-point messages into a root buffer of P*N
 // elements and a serial fold on the root (then a Bcast for Allreduce).  Here the step
-// is one grid over the element range: each lane owns U 16-byte columns, folds them over
-// the P rank buffers in rank order with D ranks' loads in flight (fold.h), and stores the
-// result to the root's buffer or to every rank's.  HBM traffic = the algorithmic bytes:
+// is one grid over the element range.  Large buffers: each lane owns U 16-byte columns, folds
+// them over the P rank buffers in rank order with D ranks' loads in flight (fold.h), and
+// stores the result to the root's buffer or to every rank's; smaller ones go through LDS.  HBM traffic = the algorithmic bytes:
 // P * N * s read, N * s (Reduce) or P * N * s (Allreduce) written.
 #pragma once
 
@@ -41,16 +41,150 @@ struct ReduceDev {
 constexpr int kReduceNarrowU = 2, kReduceNarrowD = 8;
 constexpr int kReduceWideU = 8, kReduceWideD = 4;
 
+// The elements past the last whole 16-byte column of a rank buffer (at least 16 bytes long),
+// by one workgroup of its own: a thread per rank loads the buffer's last 16 bytes, a lane per
+// element folds them from LDS.  (One wave that loads an element of rank after rank waits two
+// latencies per rank: an Allreduce on 1024 ranks took 606 us for 32769 doubles, 165 for 32768.)
+template <class T, int OP>
+__device__ __forceinline__ void reduce_tail_block(const ReduceDev& p, u32x4* s) {
+    const uint64_t bytes = (uint64_t)p.count * sizeof(T);
+    const int rem = (int)(bytes & 15), nel = rem / (int)sizeof(T), t = threadIdx.x;
+    T acc{};
+    for (int r0 = 0; r0 < p.P; r0 += kReduceThreads) {
+        if (r0 + t < p.P) s[t] = gload16(*(const uint64_t*)(p.sendbufs + 8 * (int64_t)(r0 + t)) + bytes - 16);
+        __syncthreads();
+        const int n = p.P - r0 < kReduceThreads ? p.P - r0 : kReduceThreads;
+        if (t < nel) {
+            const T* x = (const T*)((const char*)s + 16 - rem) + t;
+            for (int j = 0; j < n; j++, x += 16 / sizeof(T)) acc = r0 + j == 0 ? *x : combine<T, OP>(*x, acc);
+        }
+        __syncthreads();
+    }
+    if (t < nel) ((T*)s)[t] = acc;
+    __syncthreads();
+    const T* y = (const T*)s;
+    for (int r = t; r < p.P; r += kReduceThreads) {
+        if (p.root >= 0 && r != p.root) continue;
+        T* to = (T*)(*(const uint64_t*)(p.recvbufs + 8 * (int64_t)r) + bytes - rem);
+        for (int e = 0; e < nel; e++) to[e] = y[e];
+    }
+}
+
+// Small and middle-sized buffers: a workgroup owns a tile of C = 1 << log_cols 16-byte columns
+// of every rank buffer.  Its threads load the tile of kStagedK * 256 / C ranks at once, park
+// it in LDS, and a thread per element folds it in rank order while the next ranks' loads
+// are in flight.  A wave that folds its columns straight from HBM (the kernels below) holds
+// D ranks in flight, so P ranks cost P / D latencies on as few waves as the buffer has
+// tiles.  Bound by latency: pointer, data, then the fold's P operations.  Allreduce of doubles,
+// from HBM -> staged: 1024 ranks x 4 KiB 165 -> 24 us, 128 KiB 168 -> 52; 32 ranks x 4 KiB
+// 6.8 -> 3.2.
+constexpr int kStagedK = 8;
+
+template <class T, int OP>
+__global__ void __launch_bounds__(kReduceThreads) batched_reduce_staged_kernel(ReduceDev p, int log_cols) {
+    __shared__ u32x4 buf[kReduceThreads * kStagedK];
+    __shared__ u32x4 res[64];
+    const uint64_t bytes = (uint64_t)p.count * sizeof(T), full = bytes / 16;
+    const uint32_t rem = (uint32_t)(bytes & 15);
+    const uint64_t ncol = full + (rem ? 1 : 0);
+    const int C = 1 << log_cols, R = kReduceThreads >> log_cols;
+    const int t = threadIdx.x, col = t & (C - 1), row = t >> log_cols;
+    const int P = p.P;
+    const GPUMPI_GLOBAL uint64_t* sends = (const GPUMPI_GLOBAL uint64_t*)p.sendbufs;
+    const GPUMPI_GLOBAL uint64_t* recvs = (const GPUMPI_GLOBAL uint64_t*)p.recvbufs;
+    for (uint64_t c0 = (uint64_t)blockIdx.x * C; c0 < ncol; c0 += (uint64_t)gridDim.x * C) {
+        const uint64_t c = c0 + col < ncol ? c0 + col : c0;
+        // the partial last column is read as the buffer's last 16 bytes (fewer: element by element)
+        const uint64_t off = c < full ? 16 * c : bytes >= 16 ? bytes - 16 : 0;
+        auto load = [&](int r) {
+            const uint64_t a = sends[r < P ? r : P - 1] + off;
+            if (bytes >= 16) return gload16(a);
+            u32x4 x{0u, 0u, 0u, 0u};
+            T e[16 / sizeof(T)] = {};
+#pragma unroll
+            for (int i = 0; i < (int)(16 / sizeof(T)) - 1; i++)
+                if (i < (int)(rem / sizeof(T))) e[i] = ((const GPUMPI_GLOBAL T*)a)[i];
+            __builtin_memcpy(&x, e, 16);
+            return x;
+        };
+        const uint64_t left = (bytes - 16 * c0) / sizeof(T);
+        const int nel = (int)(left < (uint64_t)C * 16 / sizeof(T) ? left : (uint64_t)C * 16 / sizeof(T));
+        uint32_t at = (uint32_t)t * (uint32_t)sizeof(T);     // this thread's element in a rank's row
+        if (c0 + at / 16 >= full && bytes >= 16) at += 16 - rem;
+        u32x4 v[kStagedK];
+#pragma unroll
+        for (int k = 0; k < kStagedK; k++)
+            if (k * R < P) v[k] = load(row + k * R);
+        T acc{};
+        for (int r0 = 0; r0 < P; r0 += kStagedK * R) {
+#pragma unroll
+            for (int k = 0; k < kStagedK; k++)
+                if (r0 + k * R < P) buf[(row + k * R) * C + col] = v[k];
+            __syncthreads();
+            const int r1 = r0 + kStagedK * R;
+#pragma unroll
+            for (int k = 0; k < kStagedK; k++)
+                if (r1 + k * R < P) v[k] = load(r1 + row + k * R);
+            if (t < nel) {
+                const char* x = (const char*)buf + at;
+                const int n = P - r0 < kStagedK * R ? P - r0 : kStagedK * R;
+                int j = 0;
+                if (r0 == 0) {
+                    acc = *(const T*)x;
+                    j = 1;
+                }
+                for (; j + 8 <= n; j += 8) {
+                    T y[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) y[i] = *(const T*)(x + (uint32_t)(j + i) * 16u * (uint32_t)C);
+#pragma unroll
+                    for (int i = 0; i < 8; i++) acc = combine<T, OP>(y[i], acc);
+                }
+                for (; j < n; j++) acc = combine<T, OP>(*(const T*)(x + (uint32_t)j * 16u * (uint32_t)C), acc);
+            }
+            __syncthreads();
+        }
+        if (t < nel) ((T*)res)[t] = acc;
+        __syncthreads();
+        const bool mine = c0 + col < ncol, whole = c < full;
+        const u32x4 y = res[col];
+        if (mine) {
+            const int step = p.root < 0 ? R : P;
+            for (int r = p.root < 0 ? row : row == 0 ? p.root : P; r < P; r += step) {
+                const uint64_t to = recvs[r] + 16 * c;
+                if (whole) {
+                    if (p.nt) gstore16<true>(to, y);
+                    else gstore16<false>(to, y);
+                } else {
+                    T e[16 / sizeof(T)];
+                    __builtin_memcpy(e, &y, 16);
+#pragma unroll
+                    for (int i = 0; i < (int)(16 / sizeof(T)); i++)
+                        if (i < (int)(rem / sizeof(T))) ((GPUMPI_GLOBAL T*)to)[i] = e[i];
+                }
+            }
+        }
+        __syncthreads();      // res is rewritten by the next tile
+    }
+}
+
 template <class T, int OP, int U, int D>
 __global__ void __launch_bounds__(kReduceThreads) batched_reduce_kernel(ReduceDev p) {
+    __shared__ u32x4 s_tail[kReduceThreads];
+    // a last column that is not whole: the first workgroup has it
+    const uint32_t tail = (uint64_t)p.count * sizeof(T) % 16 ? 1 : 0;
+    if (blockIdx.x < tail) {
+        reduce_tail_block<T, OP>(p, s_tail);
+        return;
+    }
     const uint64_t nvec = (uint64_t)p.count * sizeof(T) / 16;
     const PtrTable src{p.sendbufs, 8}, dst{p.recvbufs, 8};
     const uint64_t one = p.root >= 0 ? *(const uint64_t*)(p.recvbufs + 8 * (int64_t)p.root) : 0;
     constexpr uint64_t kTile = (uint64_t)kWave * U;  // 16-byte columns per wave and visit
     const uint64_t ntiles = (nvec + kTile - 1) / kTile;
     const uint64_t wpb = kReduceThreads / kWave;
-    const uint64_t nw = (uint64_t)gridDim.x * wpb;
-    for (uint64_t t = (uint64_t)blockIdx.x * wpb + (threadIdx.x >> 6); t < ntiles; t += nw) {
+    const uint64_t nw = (uint64_t)(gridDim.x - tail) * wpb;
+    for (uint64_t t = (uint64_t)(blockIdx.x - tail) * wpb + (threadIdx.x >> 6); t < ntiles; t += nw) {
         const uint64_t v0 = t * kTile + (uint64_t)lane();
         uint32_t valid = 0;
 #pragma unroll
@@ -61,9 +195,6 @@ __global__ void __launch_bounds__(kReduceThreads) batched_reduce_kernel(ReduceDe
         if (p.nt) fold_store_cols<true, U>(dst, p.P, one, 16 * v0, valid, acc);
         else fold_store_cols<false, U>(dst, p.P, one, 16 * v0, valid, acc);
     }
-    // elements past the last whole 16-byte column
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x < kWave)
-        fold_scalar_tail<T, OP>(src, p.P, dst, p.P, one, (int64_t)(nvec * 16 / sizeof(T)), p.count);
 }
 
 // Integer operators are exact in any order, so below the wide shape their fold splits the
@@ -81,6 +212,12 @@ template <class T, int OP, int U, int D>
 __global__ void __launch_bounds__(kReduceThreads) batched_reduce_split_kernel(ReduceDev p) {
     constexpr int S = kReduceSplitWaves;
     __shared__ u32x4 part[S][U][kWave];
+    static_assert(S * U * kWave >= kReduceThreads, "part holds the tail's ranks");
+    const uint32_t tail = (uint64_t)p.count * sizeof(T) % 16 ? 1 : 0;
+    if (blockIdx.x < tail) {
+        reduce_tail_block<T, OP>(p, &part[0][0][0]);
+        return;
+    }
     const uint64_t nvec = (uint64_t)p.count * sizeof(T) / 16;
     constexpr uint64_t kTile = (uint64_t)kWave * U;
     const uint64_t ntiles = (nvec + kTile - 1) / kTile;
@@ -90,7 +227,7 @@ __global__ void __launch_bounds__(kReduceThreads) batched_reduce_split_kernel(Re
     const PtrTable dsub{p.recvbufs + 8 * (int64_t)r0, 8};
     const uint64_t one = p.root >= 0 ? *(const uint64_t*)(p.recvbufs + 8 * (int64_t)p.root) : 0;
     const int l = lane();
-    for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    for (uint64_t t = blockIdx.x - tail; t < ntiles; t += gridDim.x - tail) {
         const uint64_t v0 = t * kTile + (uint64_t)l;
         uint32_t valid = 0;
 #pragma unroll
@@ -118,11 +255,6 @@ __global__ void __launch_bounds__(kReduceThreads) batched_reduce_split_kernel(Re
             if (p.nt) fold_store_cols<true, U>(dsub, r1 - r0, 0, 16 * v0, valid, tot);
             else fold_store_cols<false, U>(dsub, r1 - r0, 0, 16 * v0, valid, tot);
         }
-    }
-    // elements past the last whole 16-byte column
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x < kWave) {
-        const PtrTable all{p.sendbufs, 8}, dall{p.recvbufs, 8};
-        fold_scalar_tail<T, OP>(all, p.P, dall, p.P, one, (int64_t)(nvec * 16 / sizeof(T)), p.count);
     }
 }
 
@@ -169,6 +301,28 @@ __host__ inline const void* batched_reduce_kernel_shape(int dt, int op) {
 __host__ inline const void* batched_reduce_kernel_for(int dt, int op, bool wide) {
     return wide ? batched_reduce_kernel_shape<kReduceWideU, kReduceWideD>(dt, op)
                 : batched_reduce_kernel_shape<kReduceNarrowU, kReduceNarrowD>(dt, op);
+}
+
+// The staged kernel for a (datatype, built-in operator) pair, or nullptr.
+__host__ inline const void* batched_reduce_staged_for(int dt, int op) {
+#define GPUMPI_RED_STAGED(T)                                                     \
+    switch (op) {                                                                \
+    case kOpMax: return (const void*)&batched_reduce_staged_kernel<T, kOpMax>;   \
+    case kOpMin: return (const void*)&batched_reduce_staged_kernel<T, kOpMin>;   \
+    case kOpSum: return (const void*)&batched_reduce_staged_kernel<T, kOpSum>;   \
+    case kOpProd: return (const void*)&batched_reduce_staged_kernel<T, kOpProd>; \
+    default: return nullptr;                                                     \
+    }
+    switch (dt) {
+    case MPI_INT: case MPI_INT32_T: GPUMPI_RED_STAGED(int32_t)
+    case MPI_UNSIGNED: case MPI_UINT32_T: GPUMPI_RED_STAGED(uint32_t)
+    case MPI_LONG: case MPI_LONG_LONG_INT: case MPI_LONG_LONG: case MPI_INT64_T: GPUMPI_RED_STAGED(int64_t)
+    case MPI_UNSIGNED_LONG: case MPI_UNSIGNED_LONG_LONG: case MPI_UINT64_T: GPUMPI_RED_STAGED(uint64_t)
+    case MPI_FLOAT: GPUMPI_RED_STAGED(float)
+    case MPI_DOUBLE: case MPI_LONG_DOUBLE: GPUMPI_RED_STAGED(double)
+    default: return nullptr;
+    }
+#undef GPUMPI_RED_STAGED
 }
 
 // The split kernel for an integer (datatype, built-in operator) pair, or nullptr.

@@ -26,5 +26,6 @@ const void* a2av_copy_kernel_for(int U, bool nt, bool defer, bool fuse);
 // in the narrow or wide shape, or nullptr.
 const void* batched_reduce_kernel_lookup(int dt, int op, bool wide);
 const void* batched_reduce_split_lookup(int dt, int op);
+const void* batched_reduce_staged_lookup(int dt, int op);
 
 }  // namespace gpumpi
