@@ -1310,8 +1310,8 @@ static_assert(sizeof(gpumpi_p2p_pair) == sizeof(P2pPair) && offsetof(gpumpi_p2p_
 
 struct gpumpi_p2p_plan {
     int64_t max_pairs = 0;
-    int64_t* chunk_off = nullptr;   // [max_pairs + 1]
-    int32_t grid = 0;               // copy workgroups
+    uint64_t* chunk_off = nullptr;  // [max_pairs], then the tiles' chunks [kP2pTiles]
+    int32_t cus = 0;
     hipGraphExec_t graph = nullptr;
     hipGraph_t graph_def = nullptr;
     int graph_steps = 0;
@@ -1323,9 +1323,25 @@ struct gpumpi_p2p_plan {
 // The step's two kernels on stream s (no allocation, no host synchronisation: capturable).
 static int p2p_launch(gpumpi_p2p_plan* pl, const P2pPair* pairs, int64_t n, hipStream_t s, bool timed) {
     if (timed) hipEventRecord(pl->ev[0], s);
-    p2p_scan_kernel<<<dim3(1), dim3(kP2pScanThreads), 0, s>>>(pairs, n, pl->chunk_off);
+    uint64_t* tile_chunks = pl->chunk_off + pl->max_pairs;
+    int shift = 12;    // pairs per tile: kP2pPass, or as many as leave kP2pTiles tiles
+    static_assert(1 << 12 == kP2pPass, "a tile is whole passes");
+    while ((n - 1) >> shift >= kP2pTiles) shift++;
+    if (n > kP2pFused)
+        p2p_scan_kernel<<<dim3((unsigned)(((n - 1) >> shift) + 1)), dim3(kP2pScanThreads), 0, s>>>(pairs, n, shift,
+                                                                                                pl->chunk_off, tile_chunks);
     if (timed) hipEventRecord(pl->ev[1], s);
-    p2p_copy_kernel<<<dim3((unsigned)pl->grid), dim3(kP2pThreads), 0, s>>>(pairs, n, pl->chunk_off);
+    // short lists: many small workgroups, each with a scan of its own (64 pairs of 16 MiB: 420
+    // us, one workgroup of 16 waves per CU 436); longer ones: one scan per CU (3072 pairs of
+    // 5 KiB: 9.8, small workgroups 14 to 36); lists with a scan kernel: what is resident at
+    // once (65536 pairs of 4 KiB: 127 us, one large workgroup per CU 138)
+    const unsigned cus = (unsigned)pl->cus;
+    if (n <= kP2pShort)
+        p2p_copy_kernel<kP2pShort, 256, 5><<<dim3(16 * cus), dim3(256), 0, s>>>(pairs, n, shift, pl->chunk_off, tile_chunks);
+    else if (n <= kP2pFused)
+        p2p_copy_kernel<kP2pFused, 1024, 4><<<dim3(cus), dim3(1024), 0, s>>>(pairs, n, shift, pl->chunk_off, tile_chunks);
+    else
+        p2p_copy_kernel<0, 256, 5><<<dim3(5 * cus), dim3(256), 0, s>>>(pairs, n, shift, pl->chunk_off, tile_chunks);
     if (timed) hipEventRecord(pl->ev[2], s);
     return hipGetLastError() == hipSuccess ? GPUMPI_OK : GPUMPI_E_HIP;
 }
@@ -1344,8 +1360,8 @@ static int p2p_create(int64_t max_pairs, gpumpi_p2p_plan** out) {
     if (gpumpi_device_info(&cus, nullptr, nullptr) != GPUMPI_OK || cus <= 0) return GPUMPI_E_HIP;
     gpumpi_p2p_plan* pl = new gpumpi_p2p_plan();
     pl->max_pairs = max_pairs;
-    pl->grid = 4 * cus;   // 16 waves per CU
-    if (hipMalloc((void**)&pl->chunk_off, sizeof(int64_t) * (size_t)(max_pairs + 1)) != hipSuccess) {
+    pl->cus = cus;
+    if (hipMalloc((void**)&pl->chunk_off, sizeof(uint64_t) * (size_t)(max_pairs + kP2pTiles)) != hipSuccess) {
         delete pl;
         return GPUMPI_E_NOMEM;
     }

@@ -12,12 +12,17 @@
 // Here the step needs no handshake: the pair list is the match.  Work is cut at 8 KiB
 // boundaries of each destination address ("chunks"), so every chunk's interior is
 // 16-byte aligned on the store side whatever the buffers' alignment:
-//   p2p_scan_kernel  one workgroup: exclusive prefix sum of the pairs' chunk counts;
-//   p2p_copy_kernel  every wave takes an equal, contiguous range of chunks, finds its first
-//                    pair with one 64-ary search of the offsets and walks forward; a chunk is
-//                    8 unaligned 16-byte loads per lane, all issued before its stores.
+//   p2p_scan_kernel  exclusive prefix sums of the pairs' chunk counts within tiles of pairs, a
+//                    workgroup per tile, and the tiles' totals;
+//   p2p_copy_kernel  finds the pair of a chunk by 64-ary searches of the offsets and walks
+//                    forward; a chunk is 8 unaligned 16-byte loads per lane, all issued before
+//                    its non-temporal stores.
+// Lists of up to kP2pFused pairs need no scan kernel: every copy workgroup scans the whole list
+// into LDS.  Measured, us per step: 3072 pairs of 5 KiB 14.2 -> 9.8, 65536 pairs of 4 KiB 188 ->
+// 127 (one workgroup scanned them in 50), 1000 pairs of 256 KiB 118 -> 83 (the non-temporal
+// stores), 64 pairs of 16 MiB 442 -> 420.
 // HBM traffic = 2 x the bytes of the pairs (read once, written once) + 8 B per pair of
-// offsets.
+// offsets (or 24 B per pair and CU, from the L2s).
 #pragma once
 
 #include "common.h"
@@ -35,7 +40,10 @@ constexpr int kP2pChunkShift = 13;                       // 8 KiB chunks of the 
 constexpr uint64_t kP2pChunk = 1ull << kP2pChunkShift;
 constexpr int kP2pU = (int)(kP2pChunk / 16 / kWave);     // 16-byte vectors per lane and chunk
 constexpr int kP2pScanThreads = 1024;
-constexpr int kP2pThreads = 256;
+constexpr int kP2pFused = 4096;      // pairs that every workgroup scans for itself
+constexpr int kP2pShort = 256;       // and that even small workgroups do
+constexpr int kP2pPass = 4096;       // pairs per pass of a tile's scan
+constexpr int kP2pTiles = 1024;      // tiles at most: their totals are scanned into LDS
 
 // Branch-free, so that callers can issue the loads of many pairs before using any.
 __device__ __forceinline__ uint64_t p2p_chunks(const char* dst, uint64_t bytes) {
@@ -44,68 +52,80 @@ __device__ __forceinline__ uint64_t p2p_chunks(const char* dst, uint64_t bytes) 
     return bytes ? c : 0;
 }
 
-// chunk_off[i] = chunks of pairs 0 .. i-1, for i = 0 .. n (chunk_off[n] = all chunks).
-// Passes of 7168 pairs through LDS (56 KiB): the pairs are read coalesced (pair
-// k * 1024 + t by thread t) and their chunk counts parked in LDS; thread t then scans
-// counts 7t .. 7t+6, the thread sums are scanned across the workgroup (wave scans, wave
-// totals through LDS), and the exclusive offsets go back to LDS and out to chunk_off
-// coalesced again.  With one pair
-// per thread and pass, 65536 pairs took 64 dependent passes (129 us); with 16 consecutive
-// pairs per thread the loads were uncoalesced (99 us).
-constexpr int kP2pScanPer = 7;
-constexpr int kP2pScanPass = kP2pScanThreads * kP2pScanPer;
-static __global__ __launch_bounds__(kP2pScanThreads) void p2p_scan_kernel(const P2pPair* pairs, int64_t n,
-                                                                   int64_t* chunk_off) {
-    constexpr int kWaves = kP2pScanThreads / kWave;
-    __shared__ int64_t s_c[kP2pScanPass];
-    __shared__ int64_t s_w[kWaves];
-    const int t = threadIdx.x, wv = t >> 6, l = t & 63;
-    int64_t carry = 0;
-    for (int64_t i0 = 0; i0 < n; i0 += kP2pScanPass) {
-        // a clamped index (n >= 1 here) and a masked size: no branch to sink the loads into
+// Exclusive sum of one value per thread over a workgroup of NT threads, and the total; `part`
+// holds one word per wavefront and is free after the caller's next barrier.
+template <int NT>
+__device__ __forceinline__ uint64_t p2p_block_scan(uint64_t v, uint64_t* part, uint64_t* total) {
+    constexpr int kWaves = NT / kWave;
+    const int l = lane(), w = threadIdx.x >> 6;
+    uint64_t incl = v;
 #pragma unroll
-        for (int k = 0; k < kP2pScanPer; k++) {
-            const int64_t j = i0 + (int64_t)k * kP2pScanThreads + t;
-            const P2pPair p = pairs[j < n ? j : n - 1];
-            s_c[k * kP2pScanThreads + t] = (int64_t)p2p_chunks(p.dst, j < n ? p.bytes : 0);
-        }
-        __syncthreads();
-        int64_t c[kP2pScanPer];
-        int64_t sum = 0;
-#pragma unroll
-        for (int k = 0; k < kP2pScanPer; k++) {
-            c[k] = s_c[t * kP2pScanPer + k];
-            sum += c[k];
-        }
-        int64_t incl = sum;
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const int64_t u = __shfl_up(incl, o);
-            if (l >= o) incl += u;
-        }
-        if (l == kWave - 1) s_w[wv] = incl;
-        __syncthreads();
-        int64_t before = 0, all = 0;
-        for (int u = 0; u < kWaves; u++) {
-            before += u < wv ? s_w[u] : 0;
-            all += s_w[u];
-        }
-        int64_t run = carry + before + incl - sum;
-#pragma unroll
-        for (int k = 0; k < kP2pScanPer; k++) {
-            s_c[t * kP2pScanPer + k] = run;
-            run += c[k];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < kP2pScanPer; k++) {
-            const int64_t j = i0 + (int64_t)k * kP2pScanThreads + t;
-            if (j < n) chunk_off[j] = s_c[k * kP2pScanThreads + t];
-        }
-        carry += all;
-        __syncthreads();   // s_c and s_w are rewritten by the next pass
+    for (int o = 1; o < kWave; o <<= 1) {
+        const uint64_t u = __shfl_up(incl, o);
+        if (l >= o) incl += u;
     }
-    if (t == 0) chunk_off[n] = carry;
+    if (l == kWave - 1) part[w] = incl;
+    __syncthreads();
+    uint64_t before = 0, all = 0;
+#pragma unroll
+    for (int u = 0; u < kWaves; u++) {
+        const uint64_t x = part[u];
+        before += u < w ? x : 0;
+        all += x;
+    }
+    *total = all;
+    return before + incl - v;
+}
+
+// Chunk counts of pairs [i0, i0 + PASS) below i1 to exclusive offsets in s (LDS), from
+// `carry` on; returns the carry after them.  The pairs are read coalesced and without a branch
+// (a clamped index and a masked size: under a bounds branch each load would be waited for).
+template <int NT, int PASS>
+__device__ __forceinline__ uint64_t p2p_scan_pass(const P2pPair* pairs, int64_t i0, int64_t i1, uint64_t carry,
+                                                  uint64_t* s, uint64_t* part) {
+    constexpr int kPer = PASS / NT;
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int64_t j = i0 + (int64_t)k * NT + t;
+        const P2pPair p = pairs[j < i1 ? j : i1 - 1];
+        s[k * NT + t] = p2p_chunks(p.dst, j < i1 ? p.bytes : 0);
+    }
+    __syncthreads();
+    uint64_t c[kPer], sum = 0, all;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        c[k] = s[t * kPer + k];
+        sum += c[k];
+    }
+    uint64_t run = carry + p2p_block_scan<NT>(sum, part, &all);
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        s[t * kPer + k] = run;
+        run += c[k];
+    }
+    __syncthreads();
+    return carry + all;
+}
+
+// chunk_off[i] = chunks of the pairs before i in i's tile of 1 << tile_shift pairs;
+// tile_chunks[b] = chunks of tile b.
+static __global__ __launch_bounds__(kP2pScanThreads) void p2p_scan_kernel(const P2pPair* pairs, int64_t n, int tile_shift,
+                                                               uint64_t* chunk_off, uint64_t* tile_chunks) {
+    __shared__ uint64_t s_c[kP2pPass];
+    __shared__ uint64_t s_w[kP2pScanThreads / kWave];
+    const int64_t t0 = (int64_t)blockIdx.x << tile_shift, t1 = t0 + (1ll << tile_shift) < n ? t0 + (1ll << tile_shift) : n;
+    uint64_t carry = 0;
+    for (int64_t i0 = t0; i0 < t1; i0 += kP2pPass) {
+        carry = p2p_scan_pass<kP2pScanThreads, kP2pPass>(pairs, i0, t1, carry, s_c, s_w);
+#pragma unroll
+        for (int k = 0; k < kP2pPass / kP2pScanThreads; k++) {
+            const int64_t j = i0 + (int64_t)k * kP2pScanThreads + threadIdx.x;
+            if (j < t1) chunk_off[j] = s_c[k * kP2pScanThreads + threadIdx.x];
+        }
+        __syncthreads();   // s_c is rewritten by the next pass
+    }
+    if (threadIdx.x == 0) tile_chunks[blockIdx.x] = carry;
 }
 
 // Copies dst bytes [lo, hi) from the matching source bytes (one chunk or less, so at most
@@ -128,7 +148,7 @@ __device__ __forceinline__ void p2p_copy_piece(char* dst, const char* src, uint6
 #pragma unroll
         for (int u = 0; u < kP2pU; u++) v[u] = gload16(sa + 16 * ((uint64_t)u * kWave + l));
 #pragma unroll
-        for (int u = 0; u < kP2pU; u++) gstore16<false>(a + 16 * ((uint64_t)u * kWave + l), v[u]);
+        for (int u = 0; u < kP2pU; u++) gstore16<true>(a + 16 * ((uint64_t)u * kWave + l), v[u]);
     } else {
         // every lane loads (vector 0 where it has none: in range, since nvec >= 1), only the
         // stores are conditional -- loads under a condition would leave every vector's
@@ -141,40 +161,86 @@ __device__ __forceinline__ void p2p_copy_piece(char* dst, const char* src, uint6
 #pragma unroll
         for (int u = 0; u < kP2pU; u++) {
             const uint64_t k = (uint64_t)u * kWave + l;
-            if (k < nvec) gstore16<false>(a + 16 * k, v[u]);
+            if (k < nvec) gstore16<true>(a + 16 * k, v[u]);
         }
     }
 }
 
-static __global__ __launch_bounds__(kP2pThreads) void p2p_copy_kernel(const P2pPair* pairs, int64_t n,
-                                                               const int64_t* chunk_off) {
-    if (n <= 0) return;
-    const uint64_t total = (uint64_t)chunk_off[n];
-    const uint64_t nw = (uint64_t)gridDim.x * (kP2pThreads / kWave);
-    // the wave index through readfirstlane: everything derived from it (the chunk range,
-    // the search, the pair fields) is then wave-uniform and kept in SGPRs
-    const uint64_t w = (uint64_t)blockIdx.x * (kP2pThreads / kWave) + bcast((uint32_t)(threadIdx.x >> 6));
-    const uint64_t c0 = total * w / nw, c1 = total * (w + 1) / nw;
-    if (c0 >= c1) return;
-    // the pair holding chunk c0: chunk_off[lo] <= c0 < chunk_off[hi] throughout
+// Largest i < n with at(i) <= c (at non-decreasing, at(0) <= c); wave-uniform, 64-ary.
+template <class F>
+__device__ __forceinline__ int64_t p2p_search(int64_t n, uint64_t c, F at) {
     int64_t lo = 0, hi = n;
     while (hi - lo > 1) {
         const int64_t step = (hi - lo + kWave - 1) / kWave;
         const int64_t probe = lo + (int64_t)lane() * step;
-        const bool le = probe < hi && (uint64_t)chunk_off[probe] <= c0;
+        const bool le = probe < hi && at(probe < hi ? probe : lo) <= c;
         const uint64_t m = ballot(le);                 // lane 0 (probe = lo) always holds
-        const int k = 63 - __builtin_clzll(m);
-        lo += (int64_t)k * step;
+        lo += (int64_t)(63 - __builtin_clzll(m)) * step;
         hi = lo + step < hi ? lo + step : hi;
     }
-    int64_t i = lo;
-    uint64_t next = (uint64_t)chunk_off[i + 1];
+    return lo;
+}
+
+// The copy, by workgroups of NT threads.  FUSED: n <= FUSED pairs and no scan kernel ran; s_off
+// holds every pair's first chunk.  FUSED = 0: s_off holds every tile's first chunk, and a pair's
+// is its tile's plus chunk_off.
+template <int FUSED, int NT, int WAVES>
+static __global__ __launch_bounds__(NT, WAVES) void p2p_copy_kernel(const P2pPair* pairs, int64_t n, int tile_shift,
+                                                             const uint64_t* chunk_off, const uint64_t* tile_chunks) {
+    __shared__ uint64_t s_off[FUSED ? FUSED : kP2pTiles];
+    __shared__ uint64_t s_w[NT / kWave];
+    const int64_t tiles = FUSED ? n : (n + (1ll << tile_shift) - 1) >> tile_shift;
+    uint64_t total;
+    if constexpr (FUSED != 0) {
+        total = p2p_scan_pass<NT, FUSED>(pairs, 0, n, 0, s_off, s_w);
+    } else {
+        constexpr int kPer = kP2pTiles / NT;
+        uint64_t c[kPer], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int b = (int)threadIdx.x * kPer + k;
+            c[k] = b < tiles ? tile_chunks[b] : 0;
+            sum += c[k];
+        }
+        uint64_t run = p2p_block_scan<NT>(sum, s_w, &total);
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            s_off[threadIdx.x * kPer + k] = run;
+            run += c[k];
+        }
+        __syncthreads();
+    }
+    // first chunk of pair i, i <= n
+    auto first = [&](int64_t i) -> uint64_t {
+        if (i >= n) return total;
+        if constexpr (FUSED != 0) return s_off[i];
+        else return s_off[i >> tile_shift] + chunk_off[i];
+    };
+    const uint64_t nw = (uint64_t)gridDim.x * (NT / kWave);
+    // the wave index through readfirstlane: everything derived from it (the chunk range,
+    // the search, the pair fields) is then wave-uniform and kept in SGPRs
+    const uint64_t w = (uint64_t)blockIdx.x * (NT / kWave) + bcast((uint32_t)(threadIdx.x >> 6));
+    const uint64_t c0 = total * w / nw, c1 = total * (w + 1) / nw;
+    if (c0 >= c1) return;
+    int64_t i = p2p_search(tiles, c0, [&](int64_t k) { return s_off[k]; });
+    if constexpr (FUSED == 0) {
+        const int64_t b = i << tile_shift, left = n - b;
+        const uint64_t in_tile = c0 - bcast(s_off[i]);
+        i = b + p2p_search(left < (1ll << tile_shift) ? left : 1ll << tile_shift, in_tile,
+                           [&](int64_t k) { return chunk_off[b + k]; });
+    }
+    uint64_t here = bcast(first(i)), next = bcast(first(i + 1));
+    P2pPair p = pairs[i];
     for (uint64_t c = c0; c < c1; c++) {
-        while (c >= next) next = (uint64_t)chunk_off[++i + 1];   // skips empty pairs
-        const P2pPair p = pairs[i];
+        if (c >= next) {
+            do {                                             // skips empty pairs
+                here = next;
+                next = bcast(first(++i + 1));
+            } while (c >= next);
+            p = pairs[i];
+        }
         const uint64_t d = (uint64_t)(uintptr_t)p.dst;
-        const uint64_t k = c - (uint64_t)chunk_off[i];
-        const uint64_t blk = ((d >> kP2pChunkShift) + k) << kP2pChunkShift;
+        const uint64_t blk = ((d >> kP2pChunkShift) + (c - here)) << kP2pChunkShift;
         const uint64_t plo = blk > d ? blk : d;
         const uint64_t phi = blk + kP2pChunk < d + p.bytes ? blk + kP2pChunk : d + p.bytes;
         p2p_copy_piece(p.dst, p.src, plo, phi);

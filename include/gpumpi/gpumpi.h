@@ -299,7 +299,7 @@ typedef struct gpumpi_p2p_pair {
 } gpumpi_p2p_pair;
 typedef struct gpumpi_p2p_plan gpumpi_p2p_plan;
 
-/* A plan for lists of up to max_pairs pairs (allocates 8 * (max_pairs + 1) bytes). */
+/* A plan for lists of up to max_pairs pairs (allocates 8 * max_pairs + 8192 bytes). */
 int gpumpi_p2p_plan_create(int64_t max_pairs, gpumpi_p2p_plan** out);
 void gpumpi_p2p_plan_destroy(gpumpi_p2p_plan* plan);
 /* One step over pairs[0 .. npairs) on `stream`: asynchronous, allocates nothing, may be
