@@ -509,7 +509,7 @@ static __global__ __launch_bounds__(NT, NT == 1024 ? 8 : 4) void bucket_scatter_
 // more keys than one workgroup should take (skewed keys) are counted by several workgroups
 // into a table and written by sort_part_expand.  HBM traffic 16 B per key (4 read twice, 2
 // written, 2 read, 4 written).  Measured for 2^27 uniform keys below 2^23 as the bucket
-// exchange leaves them: top_hist 108 us, split 254, part 171.  Counting with an atomic per key
+// exchange leaves them: top_hist 94 us, split 254, part 170.  Counting with an atomic per key
 // on 2^23 counters in HBM, and writing each value's run with one thread, took 4731 + 580 us.
 // Longer keys, and an output that overlaps the keys (the split would overwrite keys not
 // yet read), keep the counters in HBM (sort_hist and what follows it).
@@ -560,13 +560,39 @@ __device__ __forceinline__ uint32_t lds_count(uint32_t* lds, uint32_t b, bool va
     return place;
 }
 
-// Four keys per lane counted by their parts; one add where the whole wave has one part.
+// Whether the wave's N keys per lane (those below the lane's `live`) lie in at most two parts, a
+// and b (b = a if in one); every lane's first key must be live.
+template <int N>
+__device__ __forceinline__ bool sort_two_parts(const uint32_t (&part)[N], const bool (&live)[N], uint32_t* a, uint32_t* b) {
+    const uint32_t a0 = bcast(part[0]);
+    uint32_t other = a0;
+#pragma unroll
+    for (int i = 0; i < N; i++) other = live[i] && part[i] != a0 ? part[i] : other;
+    const uint64_t have = ballot(other != a0);
+    const uint32_t b0 = have ? readlane(other, __builtin_ctzll(have)) : a0;
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < N; i++) ok = ok && (!live[i] || part[i] == a0 || part[i] == b0);
+    *a = a0;
+    *b = b0;
+    return ballot(!ok) == 0;
+}
+
+// Four keys per lane counted by their parts; one add per part where the wave has one or two.
 __device__ __forceinline__ void sort_count_parts(uint32_t* lds, u32x4 v) {
     const uint32_t b[4] = {v.x >> kSortLowBits, v.y >> kSortLowBits, v.z >> kSortLowBits, v.w >> kSortLowBits};
-    const uint32_t b0 = bcast(b[0]);
-    const uint64_t act = ballot(true);
-    if (ballot(b[0] == b0 && b[1] == b0 && b[2] == b0 && b[3] == b0) == act) {
-        if (lane() == (int)__builtin_ctzll(act)) atomicAdd(&lds[b0], 4u * (uint32_t)__popcll(act));
+    const bool live[4] = {true, true, true, true};
+    uint32_t p, q;
+    if (sort_two_parts(b, live, &p, &q)) {
+        const uint64_t act = ballot(true);
+        uint32_t np = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) np += (uint32_t)__popcll(ballot(b[k] == p));
+        const uint32_t nq = 4u * (uint32_t)__popcll(act) - np;
+        if (lane() == (int)__builtin_ctzll(act)) {
+            atomicAdd(&lds[p], np);
+            if (nq) atomicAdd(&lds[q], nq);
+        }
     } else {
 #pragma unroll
         for (int k = 0; k < 4; k++) lds_count(lds, b[k], true);
