@@ -923,17 +923,25 @@ static int a2av_configure(gpumpi_a2av_plan* pl, const gpumpi_a2av_tune& t) {
     return GPUMPI_OK;
 }
 
-// One step of three kernels on workspace 0: plan, scan, copy.
+// Plan and scan kernels (one kernel for few ranks); ev, if given, is recorded between them.
+static int a2av_launch_tables(A2avDev& d, bool plan, hipStream_t s, hipEvent_t ev = nullptr) {
+    void* kargs[] = {(void*)&d};
+    const bool small = plan && d.P <= kA2avSmallRanks;
+    if (plan && hipLaunchKernel(small ? (const void*)&a2av_plan_small_kernel : (const void*)&a2av_plan_kernel,
+                                dim3(small ? 1 : d.P), dim3(small ? 1024 : 256), kargs, 0, s) != hipSuccess)
+        return GPUMPI_E_HIP;
+    if (ev) hipEventRecord(ev, s);
+    if (!small && hipLaunchKernel((const void*)&a2av_scan_kernel, dim3(1), dim3(1024), kargs, 0, s) != hipSuccess)
+        return GPUMPI_E_HIP;
+    return GPUMPI_OK;
+}
+
+// One step on workspace 0: plan, scan, copy.
 static int a2av_launch(gpumpi_a2av_plan* pl, hipStream_t s, bool timed) {
     A2avDev& d = pl->dev;
     void* kargs[] = {(void*)&d, (void*)&d};
-    void* kargs1[] = {(void*)&d};
     if (timed) hipEventRecord(pl->ev[0], s);
-    if (hipLaunchKernel((const void*)&a2av_plan_kernel, dim3(d.P), dim3(256), kargs1, 0, s) != hipSuccess)
-        return GPUMPI_E_HIP;
-    if (timed) hipEventRecord(pl->ev[1], s);
-    if (hipLaunchKernel((const void*)&a2av_scan_kernel, dim3(1), dim3(1024), kargs1, 0, s) != hipSuccess)
-        return GPUMPI_E_HIP;
+    if (a2av_launch_tables(d, true, s, timed ? pl->ev[1] : nullptr) != GPUMPI_OK) return GPUMPI_E_HIP;
     if (timed) hipEventRecord(pl->ev[2], s);
     if (hipLaunchKernel(a2av_copy_for(pl->tune.lines_per_lane, pl->tune.nontemporal > 0,
                                       pl->tune.defer_straddle > 0, false),
@@ -963,13 +971,7 @@ static int a2av_launch_copy(gpumpi_a2av_plan* pl, hipStream_t s, int cur, bool p
 }
 
 static int a2av_launch_plan_scan(gpumpi_a2av_plan* pl, hipStream_t s, int ws, bool plan) {
-    A2avDev& d = ws == 0 ? pl->dev : pl->dev2;
-    void* kargs1[] = {(void*)&d};
-    if (plan && hipLaunchKernel((const void*)&a2av_plan_kernel, dim3(d.P), dim3(256), kargs1, 0, s) != hipSuccess)
-        return GPUMPI_E_HIP;
-    if (hipLaunchKernel((const void*)&a2av_scan_kernel, dim3(1), dim3(1024), kargs1, 0, s) != hipSuccess)
-        return GPUMPI_E_HIP;
-    return GPUMPI_OK;
+    return a2av_launch_tables(ws == 0 ? pl->dev : pl->dev2, plan, s);
 }
 
 // `steps` steps, in the pipeline mode of the tune:
@@ -1161,12 +1163,8 @@ int gpumpi_a2av_pipeline_times(gpumpi_a2av_plan* pl, int32_t steps, void* stream
     for (hipEvent_t& e : ev)
         if (hipEventCreate(&e) != hipSuccess) return GPUMPI_E_HIP;
     int rc = GPUMPI_OK;
-    A2avDev& d = pl->dev;
-    void* kargs1[] = {(void*)&d};
     hipEventRecord(ev[0], s);
-    if (hipLaunchKernel((const void*)&a2av_plan_kernel, dim3(d.P), dim3(256), kargs1, 0, s) != hipSuccess ||
-        hipLaunchKernel((const void*)&a2av_scan_kernel, dim3(1), dim3(1024), kargs1, 0, s) != hipSuccess)
-        rc = GPUMPI_E_HIP;
+    rc = a2av_launch_tables(pl->dev, true, s);
     hipEventRecord(ev[1], s);
     const bool scan_in_plan = pl->tune.pipeline != 1;
     for (int i = 0; i < steps && rc == GPUMPI_OK; i++) {
@@ -2141,11 +2139,9 @@ int gpumpi_a2av_execute_noalloc(int32_t P, int32_t elem_bytes, void* const* send
     d.min_lines = (uint32_t)(kA2avCopyThreads * 4);
     d.straddle_blocks = 0;
     hipStream_t s = (hipStream_t)stream;
-    void* kargs1[] = {(void*)&d};
     void* kargs2[] = {(void*)&d, (void*)&d};
     // the copy grid strides over the chunks: 16 workgroups per CU
-    if (hipLaunchKernel((const void*)&a2av_plan_kernel, dim3(P), dim3(256), kargs1, 0, s) != hipSuccess ||
-        hipLaunchKernel((const void*)&a2av_scan_kernel, dim3(1), dim3(1024), kargs1, 0, s) != hipSuccess ||
+    if (a2av_launch_tables(d, true, s) != GPUMPI_OK ||
         hipLaunchKernel(a2av_copy_for(4, true, false, false), dim3(16 * cus), dim3(kA2avCopyThreads),
                         kargs2, 0, s) != hipSuccess)
         return GPUMPI_E_HIP;
