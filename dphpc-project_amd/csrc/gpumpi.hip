@@ -104,6 +104,30 @@ __global__ void clear_status_kernel(Runtime* R) {
     }
 }
 
+// A launch's argument block, passed by value: the bytes go to `dst` and the runtime points to
+// them.  (As two copies from pageable memory they cost more than the launch itself.)
+constexpr size_t kArgsByValue = 1024;
+struct ArgsBlock {
+    uint32_t words[kArgsByValue / 4];
+};
+__global__ void stage_args_kernel(Runtime* R, uint32_t* dst, uint32_t words, ArgsBlock a) {
+    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = a.words[i];
+    if (threadIdx.x == 0) R->user_args = dst;
+}
+
+// What the host reads after a run, in pinned memory.
+struct RunStatus {
+    int32_t abort_flag, exit_code;
+    ErrorRecord err;
+};
+__global__ void report_status_kernel(const Runtime* R, RunStatus* out) {
+    if (threadIdx.x == 0) {
+        out->abort_flag = R->abort_flag;
+        out->exit_code = R->exit_code;
+        out->err = R->err;
+    }
+}
+
 // Launch-local world size (plain one-launch-per-job mode): the first k ranks of the
 // runtime form MPI_COMM_WORLD; collective sequence numbers and barrier words restart.
 __global__ void resize_world_kernel(Runtime* R, int k) {
@@ -169,6 +193,8 @@ struct gpumpi_runtime {
     int stage_dev = 0;   // Runtime::copy_stage_bytes as last set on the device
     size_t max_lds_block = 65536;  // LDS bytes a workgroup may hold on this device
     IoSlot* io = nullptr;  // pinned host I/O request slots, one per rank
+    RunStatus* status = nullptr;           // pinned; written at the end of a run
+    hipEvent_t ev[2] = {nullptr, nullptr}; // around a run's rank grid
     class IoService* io_service = nullptr;
 };
 static void io_service_free(class IoService* s);
@@ -391,6 +417,9 @@ void gpumpi_runtime_destroy(gpumpi_runtime* rt) {
     for (void* p : rt->allocs) hipFree(p);
     io_service_free(rt->io_service);
     if (rt->io) hipHostFree(rt->io);
+    if (rt->status) hipHostFree(rt->status);
+    for (hipEvent_t e : rt->ev)
+        if (e) hipEventDestroy(e);
     if (rt->d_args) hipFree(rt->d_args);
     if (rt->own_stream) hipStreamDestroy(rt->own_stream);
     delete rt;
@@ -422,6 +451,14 @@ static int stage_args(gpumpi_runtime* rt, const void* args, size_t bytes, hipStr
         size_t cap = bytes < 4096 ? 4096 : bytes;
         HIP_TRY(hipMalloc(&rt->d_args, cap));
         rt->args_cap = cap;
+    }
+    if (bytes <= kArgsByValue && rt->d_args) {
+        ArgsBlock a;
+        if (bytes) std::memcpy(&a, args, bytes);
+        hipLaunchKernelGGL(stage_args_kernel, dim3(1), dim3(64), 0, s, rt->d_rt, (uint32_t*)rt->d_args,
+                           (uint32_t)((bytes + 3) / 4), a);
+        HIP_TRY(hipGetLastError());
+        return GPUMPI_OK;
     }
     if (bytes) HIP_TRY(hipMemcpyAsync(rt->d_args, args, bytes, hipMemcpyHostToDevice, s));
     const void* dp = rt->d_args;
@@ -709,20 +746,20 @@ static int run_entry(gpumpi_runtime* rt, const ProgramEntry* pe, int argc,
     int rc = stage_args(rt, args, args_bytes, s);
     if (rc != GPUMPI_OK) return rc;
     hipLaunchKernelGGL(clear_status_kernel, dim3(1), dim3(64), 0, s, rt->d_rt);
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
+    for (hipEvent_t& e : rt->ev)
+        if (!e) HIP_TRY(hipEventCreate(&e));
+    if (!rt->status) HIP_TRY(hipHostMalloc((void**)&rt->status, sizeof(RunStatus), hipHostMallocDefault));
+    const hipEvent_t e0 = rt->ev[0], e1 = rt->ev[1];
     HIP_TRY(hipEventRecord(e0, s));
     if (!rt->io_service) rt->io_service = new IoService(rt->io, rt->cfg.num_ranks);
     rt->io_service->begin();
     rc = launch_program(rt, pe, argc, d_argv, s);
     HIP_TRY(hipEventRecord(e1, s));
+    hipLaunchKernelGGL(report_status_kernel, dim3(1), dim3(64), 0, s, rt->d_rt, rt->status);
     hipError_t se = hipStreamSynchronize(s);
     rt->io_service->end();
     float ms = 0.f;
     hipEventElapsedTime(&ms, e0, e1);
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
     if (d_argv) hipFree(d_argv);
     if (d_blob) hipFree(d_blob);
     if (rc != GPUMPI_OK) return rc;
@@ -731,8 +768,7 @@ static int run_entry(gpumpi_runtime* rt, const ProgramEntry* pe, int argc,
         return GPUMPI_E_HIP;
     }
     if (elapsed_ms) *elapsed_ms = ms;
-    Runtime hr;
-    HIP_TRY(hipMemcpy(&hr, rt->d_rt, sizeof(Runtime), hipMemcpyDeviceToHost));
+    const RunStatus hr = *rt->status;
     if (hr.abort_flag) {
         char msg[160];
         std::snprintf(msg, sizeof(msg), "device error %d on rank %d (line %d, detail %d): %s",
