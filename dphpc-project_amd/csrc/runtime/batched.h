@@ -662,18 +662,23 @@ __device__ __forceinline__ void a2av_copy_short(const A2avDev& p, int64_t d, uin
     while (pos < line1) {
         const int64_t o0 = (int64_t)(pos << 4) - (int64_t)rbase;
         const int64_t o = o0 < 0 ? 0 : o0;
-        if (tid < kWave) {
-            int64_t s0 = 0;
-            if ((int64_t)se[0] <= o) s0 = wave_search_le(se, P, (uint64_t)o) + 1;
-            if (tid == 0) meta[5] = s0;
+        // (few ranks: the whole row, without a search for its first segment)
+        const bool whole = P <= kWave;
+        if (!whole) {
+            if (tid < kWave) {
+                int64_t s0 = 0;
+                if ((int64_t)se[0] <= o) s0 = wave_search_le(se, P, (uint64_t)o) + 1;
+                if (tid == 0) meta[5] = s0;
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        const int s0 = (int)bcast(meta[5]);
-        const int n = P - s0 < most ? P - s0 : most;
+        const int s0 = whole ? 0 : (int)bcast(meta[5]);
+        const int n = whole ? P : P - s0 < most ? P - s0 : most;
         for (int k = tid; k < n; k += kA2avCopyThreads) {
             const int s = s0 + k;
             const int64_t en = (int64_t)se[s], st = s > 0 ? (int64_t)se[s - 1] : 0;
-            sE[k] = (int32_t)(en - o < INT32_MAX ? en - o : INT32_MAX);
+            const int64_t e = en - o;
+            sE[k] = (int32_t)(e > INT32_MAX ? INT32_MAX : e < INT32_MIN / 2 ? INT32_MIN / 2 : e);
             sD[k] = src[s] - (rbase + (uint64_t)st);
             if (k == 0) meta[6] = st - o > INT32_MIN / 2 ? st - o : INT32_MIN / 2;
             if (k == n - 1) meta[7] = en;
@@ -799,13 +804,15 @@ __global__ void __launch_bounds__(kA2avCopyThreads) a2av_copy_kernel(A2avDev p, 
             return;
         }
     }
-    // the partial lines at the ends of the long rows: a lane each, in the first blocks
-    if constexpr (!DEFER) {
-        for (uint64_t g = (uint64_t)bid * kA2avCopyThreads + tid; g < 2 * (uint64_t)P; g += (uint64_t)nblk * kA2avCopyThreads)
-            a2av_row_end(p, (int64_t)(g >> 1), (int)(g & 1));
-    }
     const uint64_t total = p.chunk_off[P];
     const uint64_t C = (uint64_t)p.total_bytes[1];
+    // the partial lines at the ends of the long rows: a lane each, in the first blocks
+    if constexpr (!DEFER) {
+        if (total)
+            for (uint64_t g = (uint64_t)bid * kA2avCopyThreads + tid; g < 2 * (uint64_t)P;
+                 g += (uint64_t)nblk * kA2avCopyThreads)
+                a2av_row_end(p, (int64_t)(g >> 1), (int)(g & 1));
+    }
     uint64_t ch = bid - sb;
     for (; ch < total; ch += nblk - sb) {
         // ---- the chunk's row and line range
@@ -1009,17 +1016,32 @@ __global__ void __launch_bounds__(kA2avCopyThreads) a2av_copy_kernel(A2avDev p, 
         const uint64_t shorts = p.short_off[P], S = (uint64_t)p.total_bytes[2];
         for (; ch - total < shorts; ch += nblk) {
             if (tid < kWave) {
-                const int64_t d = wave_search_le(p.short_off, P, ch - total);
-                if (l == 0) {
-                    s_meta[0] = d;
-                    s_meta[1] = (int64_t)(ch - total - p.short_off[d]);
+                if (P <= kWave) {
+                    // every row's words in one round of loads
+                    const int r = l < P ? l : P - 1;
+                    const uint64_t off = p.short_off[r], base = (uint64_t)(uintptr_t)p.recvbufs[r], word = p.row_bytes[r];
+                    const int d = 63 - __builtin_clzll(ballot(l < P && off <= ch - total));
+                    if (l == d) {
+                        s_meta[0] = d;
+                        s_meta[1] = (int64_t)(ch - total - off);
+                        s_meta[2] = (int64_t)base;
+                        s_meta[3] = (int64_t)word;
+                    }
+                } else {
+                    const int64_t d = wave_search_le(p.short_off, P, ch - total);
+                    if (l == 0) {
+                        s_meta[0] = d;
+                        s_meta[1] = (int64_t)(ch - total - p.short_off[d]);
+                        s_meta[2] = (int64_t)(uintptr_t)p.recvbufs[d];
+                        s_meta[3] = (int64_t)p.row_bytes[d];
+                    }
                 }
             }
             __syncthreads();
             const int64_t d = bcast(s_meta[0]);
             const uint64_t c = (uint64_t)bcast(s_meta[1]);
-            const uint64_t rbase = (uint64_t)(uintptr_t)p.recvbufs[d];
-            const int64_t rbytes = (int64_t)(p.row_bytes[d] & ~kA2avShortRow);
+            const uint64_t rbase = (uint64_t)bcast(s_meta[2]);
+            const int64_t rbytes = (int64_t)((uint64_t)bcast(s_meta[3]) & ~kA2avShortRow);
             const uint64_t lend = (rbase + (uint64_t)rbytes + 15) >> 4;
             const uint64_t line0 = ((rbase >> 7) << 3) + c * S;
             const uint64_t line1 = line0 + S < lend ? line0 + S : lend;
