@@ -34,9 +34,10 @@
 //         at the ends of rows are a lane each in the first blocks.
 //         Rows of short segments, of elements that are not whole dwords, and small rows take
 //         a loop of their own (a2av_copy_short), in which each lane finds its line's segments.
-//         Measured (execute, us, before -> with it): 16 ranks x 3 KiB 24.0 -> 12.9; 200 ranks,
-//         48 MiB of bytes, segments of 157 B to 50 KiB 403 -> 39; 512 ranks, 64-byte segments,
-//         16 MiB 95 -> 35.
+//         Measured (execute, us, before -> with it): 16 ranks x 3 KiB 24.0 -> 12.9 (11.2 since
+//         up to 64 ranks are planned and scanned by one kernel and their tables read in one
+//         round); 200 ranks, 48 MiB of bytes, segments of 157 B to 50 KiB 403 -> 39; 512 ranks,
+//         64-byte segments, 16 MiB 95 -> 35.
 //
 // Why not one persistent kernel with a grid barrier: on gfx950 an agent-scope release or
 // acquire writes back or invalidates the XCD's L2 (buffer_wbl2 / buffer_inv sc1); a grid

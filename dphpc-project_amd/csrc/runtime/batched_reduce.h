@@ -11,8 +11,9 @@
 // elements and a serial fold on the root (then a Bcast for Allreduce).  Here the step
 // is one grid over the element range.  Large buffers: each lane owns U 16-byte columns, folds
 // them over the P rank buffers in rank order with D ranks' loads in flight (fold.h), and
-// stores the result to the root's buffer or to every rank's; smaller ones go through LDS.  HBM traffic = the algorithmic bytes:
-// P * N * s read, N * s (Reduce) or P * N * s (Allreduce) written.
+// stores the result to the root's buffer or to every rank's; smaller ones go through LDS.
+// HBM traffic = the algorithmic bytes: P * N * s read, N * s (Reduce) or P * N * s (Allreduce)
+// written.
 #pragma once
 
 #include "fold.h"
