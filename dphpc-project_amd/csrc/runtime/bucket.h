@@ -533,6 +533,16 @@ struct SortParts {
     uint32_t* tables;    // [ntables][kSortBins]
 };
 
+// Work items of a part of c keys, and the end of its item that starts at key i0 < c.  A part
+// may hold nearly 2^32 keys: a sum with `chunk` before the division or comparison would wrap,
+// and the part's last item, or the whole part, would be left out.
+__host__ __device__ __forceinline__ uint32_t sort_items(uint32_t c, uint32_t most, uint32_t chunk) {
+    return c > most ? (c - 1) / chunk + 1 : c ? 1 : 0;
+}
+__host__ __device__ __forceinline__ uint32_t sort_item_end(uint32_t i0, uint32_t c, uint32_t chunk) {
+    return c - i0 < chunk ? c : i0 + chunk;
+}
+
 static __global__ __launch_bounds__(kSortThreads) void sort_zero_kernel(uint32_t* p, uint32_t words) {
     for (uint32_t i = blockIdx.x * kSortThreads + threadIdx.x; i < words; i += gridDim.x * kSortThreads) p[i] = 0;
 }
@@ -631,7 +641,7 @@ static __global__ __launch_bounds__(kSortThreads) void sort_top_scan_kernel(Sort
     const uint32_t b = threadIdx.x;
     const uint32_t c = b < parts ? s.count[b] : 0;
     const bool big = c > most;
-    const uint32_t items = big ? (c + chunk - 1) / chunk : c ? 1 : 0;
+    const uint32_t items = sort_items(c, most, chunk);
     uint32_t all, nitem, nbig;
     const uint32_t first = block_excl_sum<kSortThreads>(c, part, &all);
     __syncthreads();
@@ -862,14 +872,14 @@ static __global__ __launch_bounds__(kSortThreads, 8) void sort_part_kernel(SortP
     const uint32_t first = s.first[b], c = s.first[b + 1] - first;
     const int32_t table = s.table[b];
     const uint32_t i0 = table < 0 ? 0 : nth * chunk;
-    const uint32_t i1 = table < 0 ? c : i0 + chunk < c ? i0 + chunk : c;
+    const uint32_t m = (table < 0 ? c : sort_item_end(i0, c, chunk)) - i0;
     const int t = threadIdx.x;
     for (int k = t; k < kSortBins; k += kSortThreads) hist[k] = 0;
     __syncthreads();
-    const uint16_t* k16 = (const uint16_t*)(out + first);
+    const uint16_t* k16 = (const uint16_t*)(out + first) + i0;
     constexpr uint32_t kLow = kSortBins - 1;
-    uint32_t i = i0 + 8u * (uint32_t)t;
-    for (; i + 8 <= i1; i += 8 * kSortThreads) {
+    uint32_t i = 8u * (uint32_t)t;
+    for (; i + 8 <= m; i += 8 * kSortThreads) {
         const u32x4 v = *(const sort_u32x4_a2*)(k16 + i);
         const uint32_t x[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -878,7 +888,7 @@ static __global__ __launch_bounds__(kSortThreads, 8) void sort_part_kernel(SortP
             atomicAdd(&hist[(x[k] >> 16) & kLow], 1u);
         }
     }
-    for (uint32_t j = i; j < i1 && j < i + 8; j++) atomicAdd(&hist[k16[j] & kLow], 1u);
+    for (uint32_t j = i; j < m && j < i + 8; j++) atomicAdd(&hist[k16[j] & kLow], 1u);
     __syncthreads();
     if (table < 0) {
         sort_write_runs(hist, kSortBins, b << kSortLowBits, out + first, 0, c, (uint16_t*)hist, part);
@@ -900,7 +910,7 @@ static __global__ __launch_bounds__(kSortThreads, 8) void sort_part_expand_kerne
     const int32_t table = s.table[b];
     if (table < 0) return;
     const uint32_t first = s.first[b], c = s.first[b + 1] - first;
-    const uint32_t i0 = nth * chunk, i1 = i0 + chunk < c ? i0 + chunk : c;
+    const uint32_t i0 = nth * chunk, i1 = sort_item_end(i0, c, chunk);
     sort_write_runs(s.tables + (uint64_t)table * kSortBins, kSortBins, b << kSortLowBits, out + first, i0, i1, marks,
                     part);
 }
