@@ -9,6 +9,7 @@
 #include "runtime/batched_reduce.h"
 #include "runtime/bucket.h"
 #include "runtime/particle_step.h"
+#include "runtime/workspace.h"
 #include "programs/workloads.h"
 #include "programs/serve.h"
 #include "../../include/gpumpi/gpumpi.h"
@@ -1742,88 +1743,46 @@ int gpumpi_particles_phase_times(gpumpi_particle_plan* pl, int32_t enable, doubl
 }  // extern "C"
 
 // ==================================================================== workspaces
-// Device memory of one synchronous call, lent from a few idle blocks: hipMalloc and hipFree
-// (which waits for the whole device) cost more than a small call's kernels.  A block has one
-// user from the constructor to the destructor, and the call has waited for its stream
-// by then, so any thread, stream or device may take it next.  At most kIdleBlocks blocks and
-// kIdleBytes in all stay idle; gpumpi_workspace_trim gives them back, and so does an allocation
-// that fails.
+// Device memory of gpumpi_bucket_plan and gpumpi_local_sort (workspace.h).  A block has one
+// user from the constructor to the destructor, and the call has waited for its stream by then,
+// so any thread or stream of the same device may take it next; after a wait that failed it is
+// freed instead.
 namespace {
+struct HipMemory {
+    static bool device(int* dev) { return hipGetDevice(dev) == hipSuccess; }
+    static void* alloc(size_t bytes) {
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    static bool free(void* p) { return hipFree(p) == hipSuccess; }
+};
+using Pool = WorkspacePool<HipMemory>;
+
 struct Workspace {
-    static constexpr size_t kIdleBlocks = 8, kIdleBytes = 64u << 20;
-    struct Block {
-        void* ptr;
-        size_t bytes;
-        int dev;
-    };
-    struct Pool {
-        std::mutex mu;
-        std::vector<Block> idle;
-        size_t bytes = 0;
-    };
     static Pool& pool() {
         static Pool* p = new Pool();   // outlives every static that may still call the library
         return *p;
     }
-    static int trim() {
-        std::vector<Block> gone;
-        {
-            std::lock_guard<std::mutex> g(pool().mu);
-            gone.swap(pool().idle);
-            pool().bytes = 0;
-        }
-        int rc = GPUMPI_OK;
-        for (const Block& b : gone)
-            if (hipFree(b.ptr) != hipSuccess) rc = GPUMPI_E_HIP;
-        return rc;
-    }
+    Pool::Block block;
+    void* ptr;
 
-    void* ptr = nullptr;
-    size_t bytes = 0;
-    int dev = -1;
-
-    explicit Workspace(size_t need) {
-        if (hipGetDevice(&dev) != hipSuccess) return;
-        bytes = 65536;
-        while (bytes < need) bytes *= 2;
-        if (need > kIdleBytes) bytes = need;     // never kept
-        {
-            std::lock_guard<std::mutex> g(pool().mu);
-            for (size_t i = 0; i < pool().idle.size(); i++) {
-                if (pool().idle[i].dev != dev || pool().idle[i].bytes != bytes) continue;
-                ptr = pool().idle[i].ptr;
-                pool().bytes -= bytes;
-                pool().idle.erase(pool().idle.begin() + (long)i);
-                return;
-            }
-        }
-        if (hipMalloc(&ptr, bytes) == hipSuccess) return;
-        (void)hipGetLastError();
-        ptr = nullptr;
-        trim();
-        if (hipMalloc(&ptr, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            ptr = nullptr;
-        }
+    explicit Workspace(size_t need) : block(pool().take(need)), ptr(block.ptr) {}
+    // Waits for the call's stream; `ok`: its launches were accepted.
+    int finish(hipStream_t s, bool ok) {
+        if (hipStreamSynchronize(s) == hipSuccess) return ok ? GPUMPI_OK : GPUMPI_E_HIP;
+        HipMemory::free(block.ptr);
+        block.ptr = nullptr;
+        return GPUMPI_E_HIP;
     }
-    ~Workspace() {
-        if (!ptr) return;
-        {
-            std::lock_guard<std::mutex> g(pool().mu);
-            if (bytes <= kIdleBytes - pool().bytes && pool().idle.size() < kIdleBlocks) {
-                pool().idle.push_back(Block{ptr, bytes, dev});
-                pool().bytes += bytes;
-                return;
-            }
-        }
-        hipFree(ptr);
-    }
+    ~Workspace() { pool().give(block); }
     Workspace(const Workspace&) = delete;
     Workspace& operator=(const Workspace&) = delete;
 };
 }  // namespace
 
-extern "C" int gpumpi_workspace_trim(void) { return Workspace::trim(); }
+extern "C" int gpumpi_workspace_trim(void) { return Workspace::pool().trim() ? GPUMPI_OK : GPUMPI_E_HIP; }
 
 // ==================================================================== bucket-sort caller
 extern "C" {
@@ -1882,10 +1841,7 @@ int gpumpi_bucket_plan(const uint32_t* keys, int32_t P, int64_t n, int32_t key_b
                           : (small ? &bucket_scatter_kernel<512, 4, 4096> : &bucket_scatter_kernel<512, 16, 4096>);
     hipLaunchKernelGGL(scatter, dim3(grid), dim3((unsigned)threads), 0, s, keys, P, n, shift, nb, tiles, tile_cnt,
                        prefix, bucket_lo, bucket_hi, key_buff1, send_counts, send_displs);
-    int rc = GPUMPI_OK;
-    if (hipGetLastError() != hipSuccess) rc = GPUMPI_E_HIP;
-    if (hipStreamSynchronize(s) != hipSuccess) rc = GPUMPI_E_HIP;
-    return rc;
+    return ws.finish(s, hipGetLastError() == hipSuccess);
 }
 
 }  // extern "C"
@@ -2370,8 +2326,7 @@ static int sort_short_keys(const uint32_t* keys, int64_t n, uint32_t bins, uint3
                        bins, hist);
     hipLaunchKernelGGL(sort_expand_kernel, dim3((unsigned)((n + outs - 1) / outs)), dim3(kSortThreads), 0, s, hist, bins,
                        n, outs, out);
-    const bool ok = hipGetLastError() == hipSuccess;
-    return hipStreamSynchronize(s) == hipSuccess && ok ? GPUMPI_OK : GPUMPI_E_HIP;
+    return ws.finish(s, hipGetLastError() == hipSuccess);
 }
 
 // Longer keys, split by their top bits into `parts` parts first.
@@ -2405,8 +2360,7 @@ static int sort_by_parts(const uint32_t* keys, int64_t n, uint32_t parts, uint32
     if (ntables)
         hipLaunchKernelGGL(sort_part_expand_kernel, dim3(items), dim3(kSortThreads), 0, s, sp, parts, (uint32_t)chunk,
                            out);
-    const bool ok = hipGetLastError() == hipSuccess;
-    return hipStreamSynchronize(s) == hipSuccess && ok ? GPUMPI_OK : GPUMPI_E_HIP;
+    return ws.finish(s, hipGetLastError() == hipSuccess);
 }
 
 extern "C" {
