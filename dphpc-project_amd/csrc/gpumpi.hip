@@ -9,6 +9,7 @@
 #include "runtime/batched_reduce.h"
 #include "runtime/bucket.h"
 #include "runtime/particle_step.h"
+#include "runtime/run_status.h"
 #include "runtime/workspace.h"
 #include "programs/workloads.h"
 #include "programs/serve.h"
@@ -116,12 +117,8 @@ __global__ void stage_args_kernel(Runtime* R, uint32_t* dst, uint32_t words, Arg
     if (threadIdx.x == 0) R->user_args = dst;
 }
 
-// What the host reads after a run, in pinned memory: Allreduce of 1000 doubles on 256 ranks, ten
-// calls, 357 -> 349 us with the arguments by value and the events kept.
-struct RunStatus {
-    int32_t abort_flag, exit_code;
-    ErrorRecord err;
-};
+// The run's status to pinned memory: Allreduce of 1000 doubles on 256 ranks, ten calls, 357 ->
+// 349 us with the arguments by value and the events kept.
 __global__ void report_status_kernel(const Runtime* R, RunStatus* out) {
     if (threadIdx.x == 0) {
         out->abort_flag = R->abort_flag;
@@ -759,10 +756,13 @@ static int run_entry(gpumpi_runtime* rt, const ProgramEntry* pe, int argc,
     HIP_TRY(hipEventRecord(e0, s));
     if (!rt->io_service) rt->io_service = new IoService(rt->io, rt->cfg.num_ranks);
     rt->io_service->begin();
+    status_arm(rt->status);
     rc = launch_program(rt, pe, argc, d_argv, s);
     HIP_TRY(hipEventRecord(e1, s));
-    hipLaunchKernelGGL(report_status_kernel, dim3(1), dim3(64), 0, s, rt->d_rt, rt->d_status);
+    void* report[] = {(void*)&rt->d_rt, (void*)&rt->d_status};
+    const hipError_t le = hipLaunchKernel((const void*)&report_status_kernel, dim3(1), dim3(64), report, 0, s);
     hipError_t se = hipStreamSynchronize(s);
+    if (se == hipSuccess) se = le;
     rt->io_service->end();
     float ms = 0.f;
     hipEventElapsedTime(&ms, e0, e1);
@@ -774,7 +774,12 @@ static int run_entry(gpumpi_runtime* rt, const ProgramEntry* pe, int argc,
         return GPUMPI_E_HIP;
     }
     if (elapsed_ms) *elapsed_ms = ms;
-    const RunStatus hr = *rt->status;
+    RunStatus hr;
+    if (!status_read(rt->status, &hr)) {
+        set_err(rt, "the run left no status");
+        rt->needs_reset = true;
+        return GPUMPI_E_HIP;
+    }
     if (hr.abort_flag) {
         char msg[160];
         std::snprintf(msg, sizeof(msg), "device error %d on rank %d (line %d, detail %d): %s",
