@@ -459,9 +459,11 @@ static int stage_args(gpumpi_runtime* rt, const void* args, size_t bytes, hipStr
     if (bytes <= kArgsByValue && rt->d_args) {
         ArgsBlock a;
         if (bytes) std::memcpy(&a, args, bytes);
-        hipLaunchKernelGGL(stage_args_kernel, dim3(1), dim3(64), 0, s, rt->d_rt, (uint32_t*)rt->d_args,
-                           (uint32_t)((bytes + 3) / 4), a);
-        HIP_TRY(hipGetLastError());
+        // (the launch's own result: hipGetLastError would also give an error of the thread's
+        // earlier calls, which is not this run's)
+        uint32_t words = (uint32_t)((bytes + 3) / 4);
+        void* kargs[] = {(void*)&rt->d_rt, (void*)&rt->d_args, (void*)&words, (void*)&a};
+        HIP_TRY(hipLaunchKernel((const void*)&stage_args_kernel, dim3(1), dim3(64), kargs, 0, s));
         return GPUMPI_OK;
     }
     if (bytes) HIP_TRY(hipMemcpyAsync(rt->d_args, args, bytes, hipMemcpyHostToDevice, s));
