@@ -1826,7 +1826,7 @@ int gpumpi_bucket_plan(const uint32_t* keys, int32_t P, int64_t n, int32_t key_b
     const bool small = (int64_t)P * ((n + 16 * threads - 1) / (16 * threads)) < 512;
     const int64_t tile_keys = (small ? 4 : 16) * threads;
     const int64_t tiles64 = (n + tile_keys - 1) / tile_keys;
-    const int64_t grid64 = (int64_t)((P + 7) / 8 * 8) * tiles64;
+    const int64_t grid64 = (P * tiles64 + 7) / 8 * 8;
     if (grid64 > INT32_MAX) return GPUMPI_E_ARG;
     const uint32_t tiles = (uint32_t)tiles64, grid = (uint32_t)grid64;
     const bool cols = P > 64;   // up to 64 ranks the splitters' workgroup sums the columns itself
