@@ -1776,6 +1776,10 @@ struct Workspace {
     void* ptr;
 
     explicit Workspace(size_t need) : block(pool().take(need)), ptr(block.ptr) {}
+    void take(size_t need) {       // again, after a failure
+        block = pool().take(need);
+        ptr = block.ptr;
+    }
     // Waits for the call's stream; `ok`: its launches were accepted.
     int finish(hipStream_t s, bool ok) {
         if (hipStreamSynchronize(s) == hipSuccess) return ok ? GPUMPI_OK : GPUMPI_E_HIP;
@@ -1809,6 +1813,18 @@ int gpumpi_gen_keys(uint32_t* keys, int32_t P, int64_t n, uint64_t seed, uint32_
     return hipGetLastError() == hipSuccess ? GPUMPI_OK : GPUMPI_E_HIP;
 }
 
+}  // extern "C"
+
+static auto bucket_scatter_for(bool narrow, bool small, bool turns) {
+    if (turns)
+        return narrow ? (small ? &bucket_scatter_kernel<1024, 4, 1024, true> : &bucket_scatter_kernel<1024, 16, 1024, true>)
+                      : (small ? &bucket_scatter_kernel<512, 4, 4096, true> : &bucket_scatter_kernel<512, 16, 4096, true>);
+    return narrow ? (small ? &bucket_scatter_kernel<1024, 4, 1024, false> : &bucket_scatter_kernel<1024, 16, 1024, false>)
+                  : (small ? &bucket_scatter_kernel<512, 4, 4096, false> : &bucket_scatter_kernel<512, 16, 4096, false>);
+}
+
+extern "C" {
+
 int gpumpi_bucket_plan(const uint32_t* keys, int32_t P, int64_t n, int32_t key_bits,
                        int32_t bucket_bits, uint32_t* key_buff1, int32_t* send_counts,
                        int32_t* send_displs, int32_t* bucket_lo, int32_t* bucket_hi,
@@ -1820,33 +1836,32 @@ int gpumpi_bucket_plan(const uint32_t* keys, int32_t P, int64_t n, int32_t key_b
     hipStream_t s = (hipStream_t)stream;
     const int nb = 1 << bucket_bits;
     const int shift = key_bits - bucket_bits;
-    // 16 keys per thread and tile; 4 where that leaves less than two workgroups per CU
-    const bool narrow = nb <= 1024;
-    const int64_t threads = narrow ? 1024 : 512;
-    const bool small = (int64_t)P * ((n + 16 * threads - 1) / (16 * threads)) < 512;
-    const int64_t tile_keys = (small ? 4 : 16) * threads;
-    const int64_t tiles64 = (n + tile_keys - 1) / tile_keys;
-    const int64_t grid64 = (P * tiles64 + 7) / 8 * 8;
-    if (grid64 > INT32_MAX) return GPUMPI_E_ARG;
-    const uint32_t tiles = (uint32_t)tiles64, grid = (uint32_t)grid64;
     const bool cols = P > 64;   // up to 64 ranks the splitters' workgroup sums the columns itself
-    const size_t cnt_words = (size_t)P * tiles * nb, pre_words = (size_t)P * (nb + 1);
-    Workspace ws(sizeof(int64_t) * nb + sizeof(uint32_t) * (cnt_words + pre_words));
+    BucketTiling t = bucket_tiling(P, n, nb, false);
+    const size_t pre_words = BucketTiling::prefix_words(P, nb);
+    auto scratch = [&] { return sizeof(int64_t) * nb + sizeof(uint32_t) * (pre_words + t.table_words(P, nb)); };
+    Workspace ws(scratch());
+    if (!ws.ptr && t.tiles > 1) {
+        t = bucket_tiling(P, n, nb, true);
+        ws.take(scratch());
+    }
     if (!ws.ptr) return GPUMPI_E_NOMEM;
+    const int64_t grid64 = ((int64_t)P * t.tiles + 7) / 8 * 8;
+    if (grid64 > INT32_MAX) return GPUMPI_E_ARG;
+    const uint32_t tiles = t.tiles, grid = (uint32_t)grid64;
     int64_t* acc = (int64_t*)ws.ptr;
     uint32_t* tile_cnt = (uint32_t*)(acc + nb);
-    uint32_t* prefix = tile_cnt + cnt_words;
+    uint32_t* prefix = tile_cnt + t.table_words(P, nb);     // no table: tile_cnt == prefix
     hipLaunchKernelGGL(bucket_tile_hist_kernel, dim3(grid), dim3(kBucketThreads), sizeof(uint32_t) * nb, s, keys, P,
-                       n, shift, nb, (uint32_t)tile_keys, tiles, tile_cnt);
+                       n, shift, nb, t.base * t.subs, tiles, tile_cnt, tiles > 1 ? nb : nb + 1);
     hipLaunchKernelGGL(bucket_rank_scan_kernel, dim3(P), dim3(kBucketThreads), 0, s, nb, tiles, tile_cnt, prefix);
     if (cols)
         hipLaunchKernelGGL(bucket_colsum_kernel, dim3((nb + kWave - 1) / kWave), dim3(kBucketThreads), 0, s, prefix, P,
                            nb, acc);
     hipLaunchKernelGGL(bucket_splitters_kernel, dim3(1), dim3(kBucketThreads), 0, s, cols ? acc : nullptr, prefix, P,
                        nb, n, bucket_lo, bucket_hi);
-    auto scatter = narrow ? (small ? &bucket_scatter_kernel<1024, 4, 1024> : &bucket_scatter_kernel<1024, 16, 1024>)
-                          : (small ? &bucket_scatter_kernel<512, 4, 4096> : &bucket_scatter_kernel<512, 16, 4096>);
-    hipLaunchKernelGGL(scatter, dim3(grid), dim3((unsigned)threads), 0, s, keys, P, n, shift, nb, tiles, tile_cnt,
+    auto scatter = bucket_scatter_for(nb <= 1024, t.small, t.subs > 1);
+    hipLaunchKernelGGL(scatter, dim3(grid), dim3(t.threads), 0, s, keys, P, n, shift, nb, tiles, t.subs, tile_cnt,
                        prefix, bucket_lo, bucket_hi, key_buff1, send_counts, send_displs);
     return ws.finish(s, hipGetLastError() == hipSuccess);
 }

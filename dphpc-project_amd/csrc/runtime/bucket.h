@@ -186,6 +186,35 @@ __device__ __forceinline__ uint32_t block_excl_sum(uint32_t v, uint32_t* part, u
     return before + inc - v;
 }
 
+// How the keys are cut: `tiles` workgroups per rank, each `subs` tiles of `base` keys one after
+// the other (16 keys per thread; 4 where that leaves less than two workgroups per CU).
+// One tile per workgroup while the table of counts (4 B per workgroup and bucket) takes at most
+// 32 MiB or an eighth of the keys; 4096 buckets would take half.  With one workgroup per rank
+// there is no table, only the ranks' prefixes: `least` asks for that, as far as a workgroup's
+// keys can be counted in 32 bits, where memory for more is not to be had.
+struct BucketTiling {
+    uint32_t threads, base, subs, tiles;
+    bool small;
+    __host__ __device__ uint64_t table_words(int P, int nb) const { return tiles > 1 ? (uint64_t)P * tiles * (uint64_t)nb : 0; }
+    __host__ __device__ static uint64_t prefix_words(int P, int nb) { return (uint64_t)P * (uint64_t)(nb + 1); }
+};
+constexpr uint64_t kBucketTableBytes = 32u << 20;
+__host__ __device__ inline BucketTiling bucket_tiling(int P, int64_t n, int nb, bool least) {
+    BucketTiling t;
+    t.threads = nb <= 1024 ? 1024 : 512;
+    t.small = (int64_t)P * ((n + 16 * t.threads - 1) / (16 * t.threads)) < 512;
+    t.base = (t.small ? 4 : 16) * t.threads;
+    const uint64_t all = ((uint64_t)n + t.base - 1) / t.base, keys = 4 * (uint64_t)P * (uint64_t)n;
+    uint64_t most = (keys / 8 > kBucketTableBytes ? keys / 8 : kBucketTableBytes) / (4 * (uint64_t)nb);   // workgroups
+    if (most > 0x7FFFFFF0u) most = 0x7FFFFFF0u;     // a grid's limit
+    const uint64_t per_rank = least || most < (uint64_t)P ? 1 : most / (uint64_t)P;
+    uint64_t subs = (all + per_rank - 1) / per_rank;
+    if (subs > 0x40000000u / t.base) subs = 0x40000000u / t.base;
+    t.subs = (uint32_t)subs;
+    t.tiles = (uint32_t)((all + subs - 1) / subs);
+    return t;
+}
+
 // Workgroup g of a grid of 8 * ceil(P * tiles / 8): workgroups are dealt to the 8 XCDs in turn,
 // so each XCD gets an eighth of all tiles in a row, and its L2 joins the pieces of a 128-byte
 // line that neighbouring tiles of a rank write.  (With whole ranks dealt to the XCDs, fewer
@@ -197,10 +226,10 @@ __host__ __device__ __forceinline__ bool bucket_tile_of(uint32_t g, int P, uint3
     return at < all;
 }
 
-// tile_cnt: [P][tiles][nb], every entry written.
+// tile_cnt: [P][tiles] rows of nb counts, `stride` words apart, every count written.
 static __global__ __launch_bounds__(kBucketThreads) void bucket_tile_hist_kernel(
     const uint32_t* keys, int P, int64_t n, int shift, int nb, uint32_t tile_keys, uint32_t tiles,
-    uint32_t* tile_cnt) {
+    uint32_t* tile_cnt, int stride) {
     extern __shared__ uint32_t lh[];
     int r;
     uint32_t tile;
@@ -227,24 +256,28 @@ static __global__ __launch_bounds__(kBucketThreads) void bucket_tile_hist_kernel
     for (; i0v < m; i0v += 4u * kBucketThreads)
         for (uint32_t j = i0v; j < m && j < i0v + 4; j++) atomicAdd(&lh[k[j] >> shift], 1u);
     __syncthreads();
-    uint32_t* o = tile_cnt + ((uint64_t)r * tiles + tile) * nb;
+    uint32_t* o = tile_cnt + ((uint64_t)r * tiles + tile) * stride;
     for (int b = threadIdx.x; b < nb; b += kBucketThreads) o[b] = lh[b];
 }
 
 // One workgroup per rank: tile_cnt[r][t][b] becomes the keys of bucket b in r's tiles before t;
-// prefix[r][b] = r's keys in buckets before b, b = 0 .. nb.
+// prefix[r][b] = r's keys in buckets before b, b = 0 .. nb.  A rank's only tile has no keys
+// before it: its counts lie in `prefix` itself (tile_cnt == prefix) and become the prefix in place.
 static __global__ __launch_bounds__(kBucketThreads) void bucket_rank_scan_kernel(int nb, uint32_t tiles,
                                                                         uint32_t* tile_cnt, uint32_t* prefix) {
     __shared__ uint32_t part[kBucketThreads / kWave];
     const int r = blockIdx.x;
-    uint32_t* row = tile_cnt + (uint64_t)r * tiles * nb;
     uint32_t* pre = prefix + (uint64_t)r * (nb + 1);
+    const bool only = tiles == 1;
+    uint32_t* row = only ? pre : tile_cnt + (uint64_t)r * tiles * nb;
     uint32_t carry = 0;
     constexpr int kU = 8;
     for (int b0 = 0; b0 < nb; b0 += kBucketThreads) {
         const int b = b0 + threadIdx.x;
         uint32_t sum = 0;
-        if (b < nb) {
+        if (only) {
+            if (b < nb) sum = row[b];
+        } else if (b < nb) {
             for (uint32_t t0 = 0; t0 < tiles; t0 += kU) {
                 uint32_t c[kU];
 #pragma unroll
@@ -385,10 +418,12 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
 // leave it in runs of one bucket, so that a wave's store covers a few lines instead of 64.
 // NBC: buckets provided for (1024 or 4096, whose per-wave counters need the LDS of half as many
 // waves).  The ballots (4 VALU instructions per bit) and HBM bound it about alike.
-template <int NT, int KPT, int NBC>
+// TURNS: the workgroup takes `subs` tiles in turn and moves its row of tile_off (of prefix, if the
+// rank has no other workgroup) on after each; apart, since the loop costs the single tile 1.5 %.
+template <int NT, int KPT, int NBC, bool TURNS>
 static __global__ __launch_bounds__(NT, NT == 1024 ? 8 : 4) void bucket_scatter_kernel(const uint32_t* keys, int P, int64_t n, int shift,
-                                                            int nb, uint32_t tiles, const uint32_t* tile_off,
-                                                            const uint32_t* prefix, const int32_t* lo,
+                                                            int nb, uint32_t tiles, uint32_t subs, uint32_t* tile_off,
+                                                            uint32_t* prefix, const int32_t* lo,
                                                             const int32_t* hi, uint32_t* out, int32_t* scounts,
                                                             int32_t* sdispls) {
     constexpr int kWaves = NT / kWave, kTile = NT * KPT, kPer = NBC / NT;
@@ -403,95 +438,107 @@ static __global__ __launch_bounds__(NT, NT == 1024 ? 8 : 4) void bucket_scatter_
     int r;
     uint32_t tile;
     if (!bucket_tile_of(blockIdx.x, P, tiles, &r, &tile)) return;
-    const int t = threadIdx.x, l = lane(), w = t >> 6;
-    const int64_t i0 = (int64_t)tile * kTile;
-    const uint32_t m = (uint32_t)(n - i0 < kTile ? n - i0 : kTile);
-    const uint32_t* k = keys + (int64_t)r * n + i0;
-    const uint32_t first = (uint32_t)(w * kWave * KPT + l);
-    uint32_t key[KPT], pos[KPT / 2] = {};   // positions: 16 bits each
-#pragma unroll
-    for (int i = 0; i < KPT; i++) {
-        const uint32_t j = first + i * kWave;
-        const uint32_t v = k[j < m ? j : 0];
-        // past the last key: the last bucket's last places, which are never stored
-        key[i] = j < m ? v : 0xFFFFFFFFu;
-    }
-    const uint32_t* pre = prefix + (uint64_t)r * (nb + 1);
+    uint32_t* pre = prefix + (uint64_t)r * (nb + 1);
+    uint32_t* off = tiles > 1 ? tile_off + ((uint64_t)r * tiles + tile) * nb : nullptr;
     if (tile == 0) {
-        for (int d = t; d < P; d += NT) {
+        for (int d = threadIdx.x; d < P; d += NT) {
             const int a = lo[d], b = hi[d];
             const bool some = a <= b;
             scounts[(int64_t)r * P + d] = some ? (int32_t)(pre[b + 1] - pre[a]) : 0;
             sdispls[(int64_t)r * P + d] = some ? (int32_t)pre[a] : (int32_t)pre[nb];
         }
     }
-    for (uint32_t z = t; z < kCnt / 4; z += NT) ((uint32_t*)pool)[z] = 0;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < KPT; i++) {
-        const uint32_t b = bucket_of(key[i], shift, NBC);
-        const uint64_t same = same_bucket<kBits>(b);
-        const uint32_t at = cnt[w][b];
-        __builtin_amdgcn_wave_barrier();
-        // every lane of a group of equal buckets stores the same count
-        cnt[w][b] = (uint16_t)(at + (uint32_t)__popcll(same));
-        __builtin_amdgcn_wave_barrier();
-        pos[i / 2] |= (at + lanes_below(same)) << (16 * (i & 1));
-        asm volatile("" : "+v"(pos[i / 2]));   // now: the masks of 16 keys kept for later would spill
-    }
-    __syncthreads();
-    // thread t: buckets t * kPer .. +kPer; their counts per wave become positions in the tile
-    uint32_t tot[kPer], sum = 0;
-#pragma unroll
-    for (int q = 0; q < kPer; q++) {
-        const int b = t * kPer + q;
-        uint32_t run = 0;
-#pragma unroll
-        for (int u = 0; u < kWaves; u++) {
-            const uint32_t c = cnt[u][b];
-            cnt[u][b] = (uint16_t)run;
-            run += c;
-        }
-        tot[q] = run;
-        sum += run;
-    }
-    uint32_t all;
-    uint32_t start = block_excl_sum<NT>(sum, part, &all);
-    const uint32_t* off = tile_off + ((uint64_t)r * tiles + tile) * nb;
-#pragma unroll
-    for (int q = 0; q < kPer; q++) {
-        const int b = t * kPer + q;
-#pragma unroll
-        for (int u = 0; u < kWaves; u++) cnt[u][b] = (uint16_t)(cnt[u][b] + start);
-        gbase[b] = b < nb ? pre[b] + off[b] - start : 0u;
-        start += tot[q];
-    }
-    __syncthreads();
-    asm volatile("" : "+s"(shift));   // recompute the buckets: kept, they would spill at 64 registers
-#pragma unroll
-    for (int i = 0; i < KPT; i++) pos[i / 2] += (uint32_t)cnt[w][bucket_of(key[i], shift, NBC)] << (16 * (i & 1));
-    __syncthreads();   // the counters' LDS takes the ordered keys
-#pragma unroll
-    for (int i = 0; i < KPT; i++)
-        ordered[pos[i / 2] >> (16 * (i & 1)) & 0xFFFFu] = key[i];
-    __syncthreads();
     uint32_t* o = out + (int64_t)r * n;
-    if (m == kTile) {
+    for (uint32_t sub = 0;; sub++) {
+        int t = threadIdx.x;
+        if constexpr (TURNS) asm volatile("" : "+v"(t));   // addresses anew for each tile: kept over the loop, they would spill
+        const int l = t & (kWave - 1), w = t >> 6;
+        const int64_t i0 = (TURNS ? (int64_t)tile * subs + sub : (int64_t)tile) * kTile;
+        const uint32_t m = (uint32_t)(n - i0 < kTile ? n - i0 : kTile);
+        const uint32_t* k = keys + (int64_t)r * n + i0;
+        const uint32_t first = (uint32_t)(w * kWave * KPT + l);
+        uint32_t key[KPT], pos[KPT / 2] = {};   // positions: 16 bits each
 #pragma unroll
         for (int i = 0; i < KPT; i++) {
-            const uint32_t p = (uint32_t)(t + i * NT);
-            const uint32_t v = ordered[p];
-            o[gbase[v >> shift] + p] = v;
+            const uint32_t j = first + i * kWave;
+            const uint32_t v = k[j < m ? j : 0];
+            // past the last key: the last bucket's last places, which are never stored
+            key[i] = j < m ? v : 0xFFFFFFFFu;
         }
-        return;
-    }
+        for (uint32_t z = t; z < kCnt / 4; z += NT) ((uint32_t*)pool)[z] = 0;
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < KPT; i++) {
-        const uint32_t p = (uint32_t)(t + i * NT);
-        if (p < m) {
-            const uint32_t v = ordered[p];
-            o[gbase[v >> shift] + p] = v;
+        for (int i = 0; i < KPT; i++) {
+            const uint32_t b = bucket_of(key[i], shift, NBC);
+            const uint64_t same = same_bucket<kBits>(b);
+            const uint32_t at = cnt[w][b];
+            __builtin_amdgcn_wave_barrier();
+            // every lane of a group of equal buckets stores the same count
+            cnt[w][b] = (uint16_t)(at + (uint32_t)__popcll(same));
+            __builtin_amdgcn_wave_barrier();
+            pos[i / 2] |= (at + lanes_below(same)) << (16 * (i & 1));
+            asm volatile("" : "+v"(pos[i / 2]));   // now: the masks of 16 keys kept for later would spill
         }
+        __syncthreads();
+        // thread t: buckets t * kPer .. +kPer; their counts per wave become positions in the tile
+        uint32_t tot[kPer], sum = 0;
+#pragma unroll
+        for (int q = 0; q < kPer; q++) {
+            const int b = t * kPer + q;
+            uint32_t run = 0;
+#pragma unroll
+            for (int u = 0; u < kWaves; u++) {
+                const uint32_t c = cnt[u][b];
+                cnt[u][b] = (uint16_t)run;
+                run += c;
+            }
+            tot[q] = run;
+            sum += run;
+        }
+        uint32_t all;
+        uint32_t start = block_excl_sum<NT>(sum, part, &all);
+        const bool more = TURNS && sub + 1 < subs && i0 + kTile < n;
+#pragma unroll
+        for (int q = 0; q < kPer; q++) {
+            const int b = t * kPer + q;
+#pragma unroll
+            for (int u = 0; u < kWaves; u++) cnt[u][b] = (uint16_t)(cnt[u][b] + start);
+            const uint32_t p0 = b < nb ? pre[b] : 0u, p1 = off && b < nb ? off[b] : 0u;
+            gbase[b] = p0 + p1 - start;
+            if (more && b < nb) {       // the next tile's keys of the bucket follow (only this workgroup reads the word)
+                if (off) off[b] = p1 + tot[q];
+                else pre[b] = p0 + tot[q];
+            }
+            start += tot[q];
+        }
+        __syncthreads();
+        asm volatile("" : "+s"(shift));   // recompute the buckets: kept, they would spill at 64 registers
+#pragma unroll
+        for (int i = 0; i < KPT; i++) pos[i / 2] += (uint32_t)cnt[w][bucket_of(key[i], shift, NBC)] << (16 * (i & 1));
+        __syncthreads();   // the counters' LDS takes the ordered keys
+#pragma unroll
+        for (int i = 0; i < KPT; i++)
+            ordered[pos[i / 2] >> (16 * (i & 1)) & 0xFFFFu] = key[i];
+        __syncthreads();
+        if (m == kTile) {
+#pragma unroll
+            for (int i = 0; i < KPT; i++) {
+                const uint32_t p = (uint32_t)(t + i * NT);
+                const uint32_t v = ordered[p];
+                o[gbase[v >> shift] + p] = v;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < KPT; i++) {
+                const uint32_t p = (uint32_t)(t + i * NT);
+                if (p < m) {
+                    const uint32_t v = ordered[p];
+                    o[gbase[v >> shift] + p] = v;
+                }
+            }
+        }
+        if (!more) return;
+        __syncthreads();     // the next tile's counters take the LDS
     }
 }
 

@@ -45,6 +45,14 @@ def test_bucket_plan_edges(P, n, key_bits, bucket_bits, kind, pkg, oracle, torch
     assert np.array_equal(sc.cpu().numpy(), e_sc) and np.array_equal(sd.cpu().numpy(), e_sd)
 
 
+# more than one tile per workgroup (tables past 32 MiB): two per workgroup, and a rank's only
+# workgroup, whose counts become the prefix in place
+@pytest.mark.parametrize("kind", ["uniform", "skewed"])
+@pytest.mark.parametrize("P,n,key_bits,bucket_bits", [(3, 6000000, 23, 12), (1100, 8193, 17, 12)])
+def test_bucket_plan_tiles_in_turn(P, n, key_bits, bucket_bits, kind, pkg, oracle, torch_gpu):
+    test_bucket_plan_edges(P, n, key_bits, bucket_bits, kind, pkg, oracle, torch_gpu)
+
+
 # one table up to 14 bits, parts of 2^14 values up to 24, counters in HBM beyond and when the
 # output overlaps the keys; tiles of 16384 keys; large parts are shared by workgroups
 @pytest.mark.parametrize("kind", ["uniform", "skewed", "equal", "sorted"])
