@@ -44,9 +44,9 @@ def link_cmd(objs, out):
     return [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", out, *objs]
 
 
-# Programs in the converter's output style, compiled as executables against the runtime
-# (each includes gpumpi/gpumpi_main.h) -- used by the tests.
-PROGRAMS = [os.path.join(ROOT, "tests", "programs", "pi_converted.hip")]
+# Executables used by the tests: a program in the converter's output style (it includes
+# gpumpi/gpumpi_main.h), and the bucket plan's kernels under tilings that a call seldom takes.
+PROGRAMS = [os.path.join(ROOT, "tests", "programs", p) for p in ("pi_converted.hip", "bucket_turns.hip")]
 
 
 def program_cmd(src, out):

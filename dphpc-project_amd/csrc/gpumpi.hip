@@ -8,6 +8,7 @@
 #include "runtime/batched.h"
 #include "runtime/batched_reduce.h"
 #include "runtime/bucket.h"
+#include "runtime/bucket_plan.h"
 #include "runtime/particle_step.h"
 #include "runtime/run_status.h"
 #include "runtime/workspace.h"
@@ -1813,18 +1814,6 @@ int gpumpi_gen_keys(uint32_t* keys, int32_t P, int64_t n, uint64_t seed, uint32_
     return hipGetLastError() == hipSuccess ? GPUMPI_OK : GPUMPI_E_HIP;
 }
 
-}  // extern "C"
-
-static auto bucket_scatter_for(bool narrow, bool small, bool turns) {
-    if (turns)
-        return narrow ? (small ? &bucket_scatter_kernel<1024, 4, 1024, true> : &bucket_scatter_kernel<1024, 16, 1024, true>)
-                      : (small ? &bucket_scatter_kernel<512, 4, 4096, true> : &bucket_scatter_kernel<512, 16, 4096, true>);
-    return narrow ? (small ? &bucket_scatter_kernel<1024, 4, 1024, false> : &bucket_scatter_kernel<1024, 16, 1024, false>)
-                  : (small ? &bucket_scatter_kernel<512, 4, 4096, false> : &bucket_scatter_kernel<512, 16, 4096, false>);
-}
-
-extern "C" {
-
 int gpumpi_bucket_plan(const uint32_t* keys, int32_t P, int64_t n, int32_t key_bits,
                        int32_t bucket_bits, uint32_t* key_buff1, int32_t* send_counts,
                        int32_t* send_displs, int32_t* bucket_lo, int32_t* bucket_hi,
@@ -1836,33 +1825,15 @@ int gpumpi_bucket_plan(const uint32_t* keys, int32_t P, int64_t n, int32_t key_b
     hipStream_t s = (hipStream_t)stream;
     const int nb = 1 << bucket_bits;
     const int shift = key_bits - bucket_bits;
-    const bool cols = P > 64;   // up to 64 ranks the splitters' workgroup sums the columns itself
     BucketTiling t = bucket_tiling(P, n, nb, false);
-    const size_t pre_words = BucketTiling::prefix_words(P, nb);
-    auto scratch = [&] { return sizeof(int64_t) * nb + sizeof(uint32_t) * (pre_words + t.table_words(P, nb)); };
-    Workspace ws(scratch());
+    Workspace ws(bucket_scratch_bytes(t, P, nb));
     if (!ws.ptr && t.tiles > 1) {
         t = bucket_tiling(P, n, nb, true);
-        ws.take(scratch());
+        ws.take(bucket_scratch_bytes(t, P, nb));
     }
     if (!ws.ptr) return GPUMPI_E_NOMEM;
-    const int64_t grid64 = ((int64_t)P * t.tiles + 7) / 8 * 8;
-    if (grid64 > INT32_MAX) return GPUMPI_E_ARG;
-    const uint32_t tiles = t.tiles, grid = (uint32_t)grid64;
-    int64_t* acc = (int64_t*)ws.ptr;
-    uint32_t* tile_cnt = (uint32_t*)(acc + nb);
-    uint32_t* prefix = tile_cnt + t.table_words(P, nb);     // no table: tile_cnt == prefix
-    hipLaunchKernelGGL(bucket_tile_hist_kernel, dim3(grid), dim3(kBucketThreads), sizeof(uint32_t) * nb, s, keys, P,
-                       n, shift, nb, t.base * t.subs, tiles, tile_cnt, tiles > 1 ? nb : nb + 1);
-    hipLaunchKernelGGL(bucket_rank_scan_kernel, dim3(P), dim3(kBucketThreads), 0, s, nb, tiles, tile_cnt, prefix);
-    if (cols)
-        hipLaunchKernelGGL(bucket_colsum_kernel, dim3((nb + kWave - 1) / kWave), dim3(kBucketThreads), 0, s, prefix, P,
-                           nb, acc);
-    hipLaunchKernelGGL(bucket_splitters_kernel, dim3(1), dim3(kBucketThreads), 0, s, cols ? acc : nullptr, prefix, P,
-                       nb, n, bucket_lo, bucket_hi);
-    auto scatter = bucket_scatter_for(nb <= 1024, t.small, t.subs > 1);
-    hipLaunchKernelGGL(scatter, dim3(grid), dim3(t.threads), 0, s, keys, P, n, shift, nb, tiles, t.subs, tile_cnt,
-                       prefix, bucket_lo, bucket_hi, key_buff1, send_counts, send_displs);
+    if (((int64_t)P * t.tiles + 7) / 8 * 8 > INT32_MAX) return GPUMPI_E_ARG;
+    bucket_plan_launch(t, keys, P, n, shift, nb, ws.ptr, key_buff1, send_counts, send_displs, bucket_lo, bucket_hi, s);
     return ws.finish(s, hipGetLastError() == hipSuccess);
 }
 

@@ -186,35 +186,6 @@ __device__ __forceinline__ uint32_t block_excl_sum(uint32_t v, uint32_t* part, u
     return before + inc - v;
 }
 
-// How the keys are cut: `tiles` workgroups per rank, each `subs` tiles of `base` keys one after
-// the other (16 keys per thread; 4 where that leaves less than two workgroups per CU).
-// One tile per workgroup while the table of counts (4 B per workgroup and bucket) takes at most
-// 32 MiB or an eighth of the keys; 4096 buckets would take half.  With one workgroup per rank
-// there is no table, only the ranks' prefixes: `least` asks for that, as far as a workgroup's
-// keys can be counted in 32 bits, where memory for more is not to be had.
-struct BucketTiling {
-    uint32_t threads, base, subs, tiles;
-    bool small;
-    __host__ __device__ uint64_t table_words(int P, int nb) const { return tiles > 1 ? (uint64_t)P * tiles * (uint64_t)nb : 0; }
-    __host__ __device__ static uint64_t prefix_words(int P, int nb) { return (uint64_t)P * (uint64_t)(nb + 1); }
-};
-constexpr uint64_t kBucketTableBytes = 32u << 20;
-__host__ __device__ inline BucketTiling bucket_tiling(int P, int64_t n, int nb, bool least) {
-    BucketTiling t;
-    t.threads = nb <= 1024 ? 1024 : 512;
-    t.small = (int64_t)P * ((n + 16 * t.threads - 1) / (16 * t.threads)) < 512;
-    t.base = (t.small ? 4 : 16) * t.threads;
-    const uint64_t all = ((uint64_t)n + t.base - 1) / t.base, keys = 4 * (uint64_t)P * (uint64_t)n;
-    uint64_t most = (keys / 8 > kBucketTableBytes ? keys / 8 : kBucketTableBytes) / (4 * (uint64_t)nb);   // workgroups
-    if (most > 0x7FFFFFF0u) most = 0x7FFFFFF0u;     // a grid's limit
-    const uint64_t per_rank = least || most < (uint64_t)P ? 1 : most / (uint64_t)P;
-    uint64_t subs = (all + per_rank - 1) / per_rank;
-    if (subs > 0x40000000u / t.base) subs = 0x40000000u / t.base;
-    t.subs = (uint32_t)subs;
-    t.tiles = (uint32_t)((all + subs - 1) / subs);
-    return t;
-}
-
 // Workgroup g of a grid of 8 * ceil(P * tiles / 8): workgroups are dealt to the 8 XCDs in turn,
 // so each XCD gets an eighth of all tiles in a row, and its L2 joins the pieces of a 128-byte
 // line that neighbouring tiles of a rank write.  (With whole ranks dealt to the XCDs, fewer

@@ -1,7 +1,7 @@
 // The bucket plan's workgroups: every tile of every rank is one workgroup's, and the XCDs (which
 // get the workgroups in turn) share them evenly, however few ranks there are.  The tilings cover
 // every rank's keys, and their tables stay within 32 MiB or an eighth of the keys.
-#include "runtime/bucket.h"
+#include "runtime/bucket_plan.h"
 
 #include <cstdio>
 #include <vector>

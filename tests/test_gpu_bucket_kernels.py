@@ -1,8 +1,12 @@
 """The bucket plan's and the local sort's kernels at the edges of their tiles and dispatch
 rules, against the oracle's bucket plan and numpy.sort (whole numbers: equal, no tolerance)."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
+from conftest import ROOT
 from oracle_py import bucket_plan
 
 pytestmark = pytest.mark.gpu
@@ -51,6 +55,13 @@ def test_bucket_plan_edges(P, n, key_bits, bucket_bits, kind, pkg, oracle, torch
 @pytest.mark.parametrize("P,n,key_bits,bucket_bits", [(3, 6000000, 23, 12), (1100, 8193, 17, 12)])
 def test_bucket_plan_tiles_in_turn(P, n, key_bits, bucket_bits, kind, pkg, oracle, torch_gpu):
     test_bucket_plan_edges(P, n, key_bits, bucket_bits, kind, pkg, oracle, torch_gpu)
+
+
+def test_bucket_plan_without_a_table(torch_gpu):
+    """The tiling for the case that memory for the table is not to be had (tests/programs/bucket_turns.hip)."""
+    exe = os.path.join(ROOT, "tests", "programs", "_build", "bucket_turns")
+    res = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert res.returncode == 0 and "all equal" in res.stdout, res.stdout + res.stderr
 
 
 # one table up to 14 bits, parts of 2^14 values up to 24, counters in HBM beyond and when the
