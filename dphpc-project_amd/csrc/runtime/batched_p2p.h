@@ -16,7 +16,7 @@
 //                    workgroup per tile, and the tiles' totals;
 //   p2p_copy_kernel  finds the pair of a chunk by 64-ary searches of the offsets and walks
 //                    forward; a chunk is 8 unaligned 16-byte loads per lane, all issued before
-//                    its non-temporal stores.
+//                    its stores.
 // Lists of up to kP2pFused pairs need no scan kernel: every copy workgroup scans the whole list
 // into LDS.  Measured, us per step: 3072 pairs of 5 KiB 14.2 -> 9.8, 65536 pairs of 4 KiB 188 ->
 // 127 (one workgroup scanned them in 50), 1000 pairs of 256 KiB 118 -> 83 (the non-temporal
@@ -128,8 +128,29 @@ static __global__ __launch_bounds__(kP2pScanThreads) void p2p_scan_kernel(const 
     if (threadIdx.x == 0) tile_chunks[blockIdx.x] = carry;
 }
 
+// What a step leaves in the caches, by its size: up to kP2pLoads bytes everything; then only what
+// it wrote, for its reader (the loads are non-temporal, so that the sent bytes do not push the
+// received ones out); from kP2pStores on nothing.  A pair of b bytes anywhere covers b / 8 KiB + 1
+// chunks on average.  Measured on three sets of buffers in turn, us for the step alone / with an
+// elementwise pass over the received bytes / with the same step back:
+//   pairs, size      all cached        stores cached        nothing       loads cached only
+//   3072, 15 MiB   11.3  18.4  23.1   13.2  20.3  25.8         -          10.9  18.8  26.9
+//   64, 40 MiB     15.2  31.7  30.7   17.3  32.0  37.4         -          15.5  35.3  37.2
+//   1000, 56 MiB   28.7  47.3  51.6   25.5  44.5  53.8         -          23.1  51.2  57.1
+//   3072, 96 MiB   48.8  85.0  94.3   44.0  77.6  81.5         -          43.4  83.1  94.2
+//   64, 256 MiB     107   199   213    108   192   186         -           102   208   205
+//   64, 512 MiB     211   397   421    215   397   429         -           204   400   407
+//   64, 768 MiB     319   598    -            -           313  593  626    314   604   629
+enum P2pCaching : int { kP2pCached = 0, kP2pKeepStores = 1, kP2pKeepNothing = 2 };
+constexpr uint64_t kP2pLoads = 48u << 20, kP2pStores = 512u << 20;
+__host__ __device__ __forceinline__ P2pCaching p2p_caching(uint64_t chunks, int64_t pairs) {
+    if (chunks < (kP2pLoads >> kP2pChunkShift) + (uint64_t)pairs) return kP2pCached;
+    return chunks < (kP2pStores >> kP2pChunkShift) + (uint64_t)pairs ? kP2pKeepStores : kP2pKeepNothing;
+}
+
 // Copies dst bytes [lo, hi) from the matching source bytes (one chunk or less, so at most
 // kP2pU vectors per lane).  All 64 lanes call with the same arguments.
+template <int C>
 __device__ __forceinline__ void p2p_copy_piece(char* dst, const char* src, uint64_t lo, uint64_t hi) {
     const int l = lane();
     const uint64_t d0 = (uint64_t)(uintptr_t)dst;
@@ -143,12 +164,14 @@ __device__ __forceinline__ void p2p_copy_piece(char* dst, const char* src, uint6
     if ((uint64_t)l < hi - b) *(char*)(uintptr_t)(b + l) = src[b + l - d0];
     const uint64_t nvec = (b - a) >> 4;
     const uint64_t sa = (uint64_t)(uintptr_t)src + (a - d0);
+    auto load = [](uint64_t at) { return C == kP2pCached ? gload16(at) : gload16_nt(at); };
+    constexpr bool kNt = C == kP2pKeepNothing;
     u32x4 v[kP2pU];
     if (nvec == (uint64_t)kWave * kP2pU) {
 #pragma unroll
-        for (int u = 0; u < kP2pU; u++) v[u] = gload16(sa + 16 * ((uint64_t)u * kWave + l));
+        for (int u = 0; u < kP2pU; u++) v[u] = load(sa + 16 * ((uint64_t)u * kWave + l));
 #pragma unroll
-        for (int u = 0; u < kP2pU; u++) gstore16<true>(a + 16 * ((uint64_t)u * kWave + l), v[u]);
+        for (int u = 0; u < kP2pU; u++) gstore16<kNt>(a + 16 * ((uint64_t)u * kWave + l), v[u]);
     } else {
         // every lane loads (vector 0 where it has none: in range, since nvec >= 1), only the
         // stores are conditional -- loads under a condition would leave every vector's
@@ -156,12 +179,12 @@ __device__ __forceinline__ void p2p_copy_piece(char* dst, const char* src, uint6
 #pragma unroll
         for (int u = 0; u < kP2pU; u++) {
             const uint64_t k = (uint64_t)u * kWave + l;
-            v[u] = gload16(sa + 16 * (k < nvec ? k : 0));
+            v[u] = load(sa + 16 * (k < nvec ? k : 0));
         }
 #pragma unroll
         for (int u = 0; u < kP2pU; u++) {
             const uint64_t k = (uint64_t)u * kWave + l;
-            if (k < nvec) gstore16<true>(a + 16 * k, v[u]);
+            if (k < nvec) gstore16<kNt>(a + 16 * k, v[u]);
         }
     }
 }
@@ -179,6 +202,27 @@ __device__ __forceinline__ int64_t p2p_search(int64_t n, uint64_t c, F at) {
         hi = lo + step < hi ? lo + step : hi;
     }
     return lo;
+}
+
+// Chunks [c0, c1), c0 in pair i; first(j) = pair j's first chunk.
+template <int C, class F>
+__device__ __forceinline__ void p2p_copy_chunks(const P2pPair* pairs, int64_t i, uint64_t c0, uint64_t c1, F first) {
+    uint64_t here = bcast(first(i)), next = bcast(first(i + 1));
+    P2pPair p = pairs[i];
+    for (uint64_t c = c0; c < c1; c++) {
+        if (c >= next) {
+            do {                                             // skips empty pairs
+                here = next;
+                next = bcast(first(++i + 1));
+            } while (c >= next);
+            p = pairs[i];
+        }
+        const uint64_t d = (uint64_t)(uintptr_t)p.dst;
+        const uint64_t blk = ((d >> kP2pChunkShift) + (c - here)) << kP2pChunkShift;
+        const uint64_t plo = blk > d ? blk : d;
+        const uint64_t phi = blk + kP2pChunk < d + p.bytes ? blk + kP2pChunk : d + p.bytes;
+        p2p_copy_piece<C>(p.dst, p.src, plo, phi);
+    }
 }
 
 // The copy, by workgroups of NT threads.  FUSED: n <= FUSED pairs and no scan kernel ran; s_off
@@ -229,22 +273,11 @@ static __global__ __launch_bounds__(NT, WAVES) void p2p_copy_kernel(const P2pPai
         i = b + p2p_search(left < (1ll << tile_shift) ? left : 1ll << tile_shift, in_tile,
                            [&](int64_t k) { return chunk_off[b + k]; });
     }
-    uint64_t here = bcast(first(i)), next = bcast(first(i + 1));
-    P2pPair p = pairs[i];
-    for (uint64_t c = c0; c < c1; c++) {
-        if (c >= next) {
-            do {                                             // skips empty pairs
-                here = next;
-                next = bcast(first(++i + 1));
-            } while (c >= next);
-            p = pairs[i];
-        }
-        const uint64_t d = (uint64_t)(uintptr_t)p.dst;
-        const uint64_t blk = ((d >> kP2pChunkShift) + (c - here)) << kP2pChunkShift;
-        const uint64_t plo = blk > d ? blk : d;
-        const uint64_t phi = blk + kP2pChunk < d + p.bytes ? blk + kP2pChunk : d + p.bytes;
-        p2p_copy_piece(p.dst, p.src, plo, phi);
-    }
+    // a loop each: with the choice at each store, the compiler makes one cached store of both kinds
+    const P2pCaching kind = p2p_caching(bcast(total), n);
+    if (kind == kP2pCached) p2p_copy_chunks<kP2pCached>(pairs, i, c0, c1, first);
+    else if (kind == kP2pKeepStores) p2p_copy_chunks<kP2pKeepStores>(pairs, i, c0, c1, first);
+    else p2p_copy_chunks<kP2pKeepNothing>(pairs, i, c0, c1, first);
 }
 
 }  // namespace gpumpi

@@ -22,6 +22,10 @@ typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
 __device__ __forceinline__ u32x4 gload16(uint64_t a) {
     return *(const GPUMPI_GLOBAL u32x4_a1*)(uintptr_t)a;
 }
+// The same past the caches: data that nothing reads again soon.
+__device__ __forceinline__ u32x4 gload16_nt(uint64_t a) {
+    return __builtin_nontemporal_load((const GPUMPI_GLOBAL u32x4_a1*)(uintptr_t)a);
+}
 template <bool NT>
 __device__ __forceinline__ void gstore16(uint64_t a, u32x4 v) {
     GPUMPI_GLOBAL u32x4* p = (GPUMPI_GLOBAL u32x4*)(uintptr_t)a;
