@@ -76,7 +76,8 @@ __device__ __forceinline__ void reduce_tail_block(const ReduceDev& p, u32x4* s) 
 // it in LDS, and a thread per element folds it in rank order while the next ranks' loads
 // are in flight.  A wave that folds its columns straight from HBM (the kernels below) holds
 // D ranks in flight, so P ranks cost P / D latencies on as few waves as the buffer has
-// tiles.  Bound by latency: pointer, data, then the fold's P operations.  Allreduce of doubles,
+// tiles.  Results are stored through the caches whatever their size (p.nt is the other kernels').
+// Bound by latency: pointer, data, then the fold's P operations.  Allreduce of doubles,
 // from HBM -> staged: 1024 ranks x 4 KiB 165 -> 24 us, 128 KiB 168 -> 52; 32 ranks x 4 KiB
 // 6.8 -> 3.2.
 constexpr int kStagedK = 8;
@@ -154,8 +155,7 @@ __global__ void __launch_bounds__(kReduceThreads) batched_reduce_staged_kernel(R
             for (int r = p.root < 0 ? row : row == 0 ? p.root : P; r < P; r += step) {
                 const uint64_t to = recvs[r] + 16 * c;
                 if (whole) {
-                    if (p.nt) gstore16<true>(to, y);
-                    else gstore16<false>(to, y);
+                    gstore16<false>(to, y);
                 } else {
                     T e[16 / sizeof(T)];
                     __builtin_memcpy(e, &y, 16);
