@@ -453,7 +453,7 @@ struct A2avSegView {
 
 // Segment holding row offset q (0 <= q < row bytes), by binary search over the row's
 // segment ends in HBM (the path for lines outside the LDS window).
-__device__ __forceinline__ A2avSegView a2av_seg_global(const A2avDev& p, int64_t d, uint64_t rbase,
+__host__ __device__ __forceinline__ A2avSegView a2av_seg_global(const A2avDev& p, int64_t d, uint64_t rbase,
                                                        int64_t q) {
     const uint64_t* se = p.seg_end + d * p.P;
     int64_t lo = 0, hi = p.P - 1;  // first s with se[s] > q
@@ -495,8 +495,17 @@ __device__ __forceinline__ A2avSegView a2av_seg_at(const A2avDev& p, int64_t d, 
     return a2av_seg_global(p, d, rbase, q);
 }
 
+// Bytes at .. at + 3 (at & 3) of the 8 bytes lo, hi.
+__host__ __device__ __forceinline__ uint32_t byte_funnel(uint32_t hi, uint32_t lo, uint32_t at) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return (uint32_t)__builtin_amdgcn_alignbyte(hi, lo, at);
+#else
+    return (uint32_t)(((uint64_t)hi << 32 | lo) >> (8 * (at & 3)));
+#endif
+}
+
 // 16 bytes from byte `at` (0..16) of the 32 bytes a, b.
-__device__ __forceinline__ u32x4 bytes_from(u32x4 a, u32x4 b, uint32_t at) {
+__host__ __device__ __forceinline__ u32x4 bytes_from(u32x4 a, u32x4 b, uint32_t at) {
     const bool h16 = at & 16, h8 = at & 8, h4 = at & 4;
     // (scalars: an array would be indexed in scratch memory)
     uint32_t x0 = h16 ? b.x : a.x, x1 = h16 ? b.y : a.y, x2 = h16 ? b.z : a.z, x3 = h16 ? b.w : a.w;
@@ -512,12 +521,11 @@ __device__ __forceinline__ u32x4 bytes_from(u32x4 a, u32x4 b, uint32_t at) {
     x2 = h4 ? x3 : x2;
     x3 = h4 ? x4 : x3;
     x4 = h4 ? x5 : x4;
-    return u32x4{(uint32_t)__builtin_amdgcn_alignbyte(x1, x0, at), (uint32_t)__builtin_amdgcn_alignbyte(x2, x1, at),
-                 (uint32_t)__builtin_amdgcn_alignbyte(x3, x2, at), (uint32_t)__builtin_amdgcn_alignbyte(x4, x3, at)};
+    return u32x4{byte_funnel(x1, x0, at), byte_funnel(x2, x1, at), byte_funnel(x3, x2, at), byte_funnel(x4, x3, at)};
 }
 
 // Bytes [0, n) at address a, n < 16, in the low bytes; reads nothing else.
-__device__ __forceinline__ u32x4 load_bytes(uint64_t a, uint32_t n) {
+__host__ __device__ __forceinline__ u32x4 load_bytes(uint64_t a, uint32_t n) {
     typedef uint64_t u64_a1 __attribute__((aligned(1)));
     typedef uint32_t u32_a1 __attribute__((aligned(1)));
     typedef uint16_t u16_a1 __attribute__((aligned(1)));
@@ -546,7 +554,7 @@ __device__ __forceinline__ u32x4 load_bytes(uint64_t a, uint32_t n) {
 // read and written.  A byte at a time -- a search, a load and a store for each of 16 -- such lines took
 // most of a copy of short unaligned segments.
 template <class F>
-__device__ __forceinline__ void a2av_assemble_line(uint64_t rbase, int64_t rbytes, uint64_t line, F at) {
+__host__ __device__ __forceinline__ void a2av_assemble_line(uint64_t rbase, int64_t rbytes, uint64_t line, F at) {
     const uint64_t la = line << 4;
     const int64_t off = (int64_t)la - (int64_t)rbase;
     const int b0 = off >= 0 ? 0 : off <= -16 ? 16 : (int)-off;
@@ -630,7 +638,7 @@ __device__ void a2av_boundary_line(const A2avDev& p, int64_t d, uint64_t rbase, 
 // The first (which = 0) or last line of long row d, if it holds bytes of the row and others.
 // (Left to the copy loop, whose lane assembles it byte by byte, such a line holds up the
 // workgroup that ends its row by some 20 us.)
-__device__ __forceinline__ void a2av_row_end(const A2avDev& p, int64_t d, int which) {
+__host__ __device__ __forceinline__ void a2av_row_end(const A2avDev& p, int64_t d, int which) {
     const uint64_t word = p.row_bytes[d];
     if (word == 0 || (word & kA2avShortRow)) return;
     const uint64_t rbase = (uint64_t)(uintptr_t)p.recvbufs[d], rend = rbase + word;
@@ -641,20 +649,43 @@ __device__ __forceinline__ void a2av_row_end(const A2avDev& p, int64_t d, int wh
                        [&](int64_t q) { return a2av_seg_global(p, d, rbase, q); });
 }
 
+// The threads of a workgroup, as a2av_copy_short uses them (a test on the CPU runs them one after
+// the other).
+struct A2avGroup {
+    // f by every thread, then a barrier
+    template <class F>
+    static __device__ __forceinline__ void each(F f) {
+        f((int)threadIdx.x);
+        __syncthreads();
+    }
+    static __device__ __forceinline__ int32_t uniform(int32_t v) { return bcast(v); }
+    static __device__ __forceinline__ int64_t uniform(int64_t v) { return bcast(v); }
+    // first of the n entries of se that is above o; `slot` in LDS
+    static __device__ __forceinline__ int64_t first_above(const uint64_t* se, int64_t n, int64_t o, int64_t* slot) {
+        each([&](int tid) {
+            if (tid < kWave) {
+                int64_t s0 = 0;
+                if ((int64_t)se[0] <= o) s0 = wave_search_le(se, n, (uint64_t)o) + 1;
+                if (tid == 0) *slot = s0;
+            }
+        });
+        return bcast(*slot);
+    }
+};
+
 // Lines [pos, line1) of a row of short segments, by the whole workgroup.  Windows of up
 // to 512 segments in LDS (offsets relative to the window's first row byte `o`); each lane finds the
-// segment of its line by bisection, four lines at a time, so that the searches' LDS reads and
+// segment of its line by bisection, two lines at a time, so that the searches' LDS reads and
 // the lines' loads overlap.  A line across one boundary takes the 16 bytes up to the
 // boundary and the 16 from it, and a funnel shift; other lines are assembled piece by piece.
 // A wave-uniform cursor over the segments (the loop for long segments) gains nothing when
 // every slice of 64 lines crosses several.
-template <bool NT>
-__device__ __forceinline__ void a2av_copy_short(const A2avDev& p, int64_t d, uint64_t rbase, int64_t rbytes,
+template <bool NT, class Group>
+__host__ __device__ __forceinline__ void a2av_copy_short(const A2avDev& p, int64_t d, uint64_t rbase, int64_t rbytes,
                                                 uint64_t pos, uint64_t line1, int32_t* sE, uint64_t* sD,
                                                 int64_t* meta) {
     constexpr int U = 2;
     const int P = p.P;
-    const int tid = threadIdx.x;
     const uint64_t* se = p.seg_end + d * P;
     const uint64_t* src = p.seg_src + d * P;
     // twice the segments that a chunk of the row holds on average
@@ -665,36 +696,30 @@ __device__ __forceinline__ void a2av_copy_short(const A2avDev& p, int64_t d, uin
         const int64_t o = o0 < 0 ? 0 : o0;
         // (few ranks: the whole row, without a search for its first segment)
         const bool whole = P <= kWave;
-        if (!whole) {
-            if (tid < kWave) {
-                int64_t s0 = 0;
-                if ((int64_t)se[0] <= o) s0 = wave_search_le(se, P, (uint64_t)o) + 1;
-                if (tid == 0) meta[5] = s0;
-            }
-            __syncthreads();
-        }
-        const int s0 = whole ? 0 : (int)bcast(meta[5]);
+        const int s0 = whole ? 0 : (int)Group::first_above(se, P, o, &meta[5]);
         const int n = whole ? P : P - s0 < most ? P - s0 : most;
-        for (int k = tid; k < n; k += kA2avCopyThreads) {
-            const int s = s0 + k;
-            const int64_t en = (int64_t)se[s], st = s > 0 ? (int64_t)se[s - 1] : 0;
-            const int64_t e = en - o;
-            sE[k] = (int32_t)(e > INT32_MAX ? INT32_MAX : e < INT32_MIN / 2 ? INT32_MIN / 2 : e);
-            sD[k] = src[s] - (rbase + (uint64_t)st);
-            if (k == 0) meta[6] = st - o > INT32_MIN / 2 ? st - o : INT32_MIN / 2;
-            if (k == n - 1) meta[7] = en;
-        }
-        __syncthreads();
-        const int32_t start0 = (int32_t)bcast(meta[6]);
-        const int64_t cover = bcast(meta[7]);
+        Group::each([&](int tid) {
+            for (int k = tid; k < n; k += kA2avCopyThreads) {
+                const int s = s0 + k;
+                const int64_t en = (int64_t)se[s], st = s > 0 ? (int64_t)se[s - 1] : 0;
+                const int64_t e = en - o;
+                sE[k] = (int32_t)(e > INT32_MAX ? INT32_MAX : e < INT32_MIN / 2 ? INT32_MIN / 2 : e);
+                sD[k] = src[s] - (rbase + (uint64_t)st);
+                if (k == 0) meta[6] = st - o > INT32_MIN / 2 ? st - o : INT32_MIN / 2;
+                if (k == n - 1) meta[7] = en;
+            }
+        });
+        const int32_t start0 = (int32_t)Group::uniform(meta[6]);
+        const int64_t cover = Group::uniform(meta[7]);
         // lines inside the window's coverage; to the row's end when the window reaches it
         uint64_t pend = s0 + n >= P ? line1 : (rbase + (uint64_t)cover) >> 4;
         if (pend > line1) pend = line1;
         if (pend <= pos) {     // more segments in one line than the window holds
-            if (tid == 0)
-                a2av_assemble_line(rbase, rbytes, pos, [&](int64_t q) { return a2av_seg_global(p, d, rbase, q); });
+            Group::each([&](int tid) {
+                if (tid == 0)
+                    a2av_assemble_line(rbase, rbytes, pos, [&](int64_t q) { return a2av_seg_global(p, d, rbase, q); });
+            });
             pos++;
-            __syncthreads();
             continue;
         }
         const int top = n > 1 ? 1 << (31 - __builtin_clz(n - 1)) : 0;
@@ -704,70 +729,71 @@ __device__ __forceinline__ void a2av_copy_short(const A2avDev& p, int64_t d, uin
                 if (k + b <= n - 1 && sE[k + b - 1] <= q) k += b;
             return k;
         };
-        for (uint64_t base = pos; base < pend; base += (uint64_t)kA2avCopyThreads * U) {
-            int32_t q[U];      // window offset of the line's first row byte
-            int k[U], kind[U]; // 0 none, 1 one segment, 2 two segments, 3 assemble
-            uint32_t cut[U];
-            u32x4 v[U], w[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const uint64_t line = base + (uint64_t)u * kA2avCopyThreads + tid;
-                const int64_t off = (int64_t)(line << 4) - (int64_t)rbase;
-                kind[u] = line < pend && off > -16 ? off < 0 || off + 16 > rbytes ? 3 : 1 : 0;
-                q[u] = kind[u] ? (int32_t)(off - o) : 0;
-                if (q[u] < 0) q[u] = 0;
-                k[u] = 0;
-            }
-            for (int b = top; b > 0; b >>= 1) {
+        Group::each([&](int tid) {
+            for (uint64_t base = pos; base < pend; base += (uint64_t)kA2avCopyThreads * U) {
+                int32_t q[U];      // window offset of the line's first row byte
+                int k[U], kind[U]; // 0 none, 1 one segment, 2 two segments, 3 assemble
+                uint32_t cut[U];
+                u32x4 v[U], w[U];
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const int at = k[u] + b <= n - 1 ? k[u] + b : 0;
-                    if (at && sE[at - 1] <= q[u]) k[u] = at;
+                    const uint64_t line = base + (uint64_t)u * kA2avCopyThreads + tid;
+                    const int64_t off = (int64_t)(line << 4) - (int64_t)rbase;
+                    kind[u] = line < pend && off > -16 ? off < 0 || off + 16 > rbytes ? 3 : 1 : 0;
+                    q[u] = kind[u] ? (int32_t)(off - o) : 0;
+                    if (q[u] < 0) q[u] = 0;
+                    k[u] = 0;
+                }
+                for (int b = top; b > 0; b >>= 1) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const int at = k[u] + b <= n - 1 ? k[u] + b : 0;
+                        if (at && sE[at - 1] <= q[u]) k[u] = at;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    if (kind[u] != 1) continue;
+                    const uint64_t la = (base + (uint64_t)u * kA2avCopyThreads + tid) << 4;
+                    const int32_t e = sE[k[u]];
+                    if (e - q[u] >= 16) {
+                        v[u] = gload16(la + sD[k[u]]);
+                        continue;
+                    }
+                    // the next non-empty segment; the one after the line's last byte at most
+                    int k2 = k[u] + 1;
+                    while (k2 < n - 1 && sE[k2] <= e) k2++;
+                    const int32_t st = k[u] > 0 ? sE[k[u] - 1] : start0;
+                    if (k2 < n && sE[k2] - e >= 16 && e - st >= 16) {
+                        const uint32_t a = (uint32_t)(e - q[u]);       // bytes from the first segment
+                        v[u] = gload16(la + a - 16 + sD[k[u]]);
+                        w[u] = gload16(la + a + sD[k2]);
+                        cut[u] = 16 - a;
+                        kind[u] = 2;
+                    } else {
+                        kind[u] = 3;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const uint64_t la = (base + (uint64_t)u * kA2avCopyThreads + tid) << 4;
+                    if (kind[u] == 2) v[u] = bytes_from(v[u], w[u], cut[u]);
+                    if (kind[u] == 1 || kind[u] == 2) gstore16<NT>(la, v[u]);
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    if (kind[u] != 3) continue;
+                    a2av_assemble_line(rbase, rbytes, base + (uint64_t)u * kA2avCopyThreads + tid, [&](int64_t x) {
+                        const int j = find((int32_t)(x - o));
+                        A2avSegView g;
+                        g.st = o + (j > 0 ? sE[j - 1] : start0);
+                        g.en = o + sE[j];
+                        g.D = sD[j];
+                        return g;
+                    });
                 }
             }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (kind[u] != 1) continue;
-                const uint64_t la = (base + (uint64_t)u * kA2avCopyThreads + tid) << 4;
-                const int32_t e = sE[k[u]];
-                if (e - q[u] >= 16) {
-                    v[u] = gload16(la + sD[k[u]]);
-                    continue;
-                }
-                // the next non-empty segment; the one after the line's last byte at most
-                int k2 = k[u] + 1;
-                while (k2 < n - 1 && sE[k2] <= e) k2++;
-                const int32_t st = k[u] > 0 ? sE[k[u] - 1] : start0;
-                if (k2 < n && sE[k2] - e >= 16 && e - st >= 16) {
-                    const uint32_t a = (uint32_t)(e - q[u]);       // bytes from the first segment
-                    v[u] = gload16(la + a - 16 + sD[k[u]]);
-                    w[u] = gload16(la + a + sD[k2]);
-                    cut[u] = 16 - a;
-                    kind[u] = 2;
-                } else {
-                    kind[u] = 3;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const uint64_t la = (base + (uint64_t)u * kA2avCopyThreads + tid) << 4;
-                if (kind[u] == 2) v[u] = bytes_from(v[u], w[u], cut[u]);
-                if (kind[u] == 1 || kind[u] == 2) gstore16<NT>(la, v[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (kind[u] != 3) continue;
-                a2av_assemble_line(rbase, rbytes, base + (uint64_t)u * kA2avCopyThreads + tid, [&](int64_t x) {
-                    const int j = find((int32_t)(x - o));
-                    A2avSegView g;
-                    g.st = o + (j > 0 ? sE[j - 1] : start0);
-                    g.en = o + sE[j];
-                    g.D = sD[j];
-                    return g;
-                });
-            }
-        }
-        __syncthreads();
+        });
         pos = pend;
     }
 }
@@ -1046,7 +1072,7 @@ __global__ void __launch_bounds__(kA2avCopyThreads) a2av_copy_kernel(A2avDev p, 
             const uint64_t lend = (rbase + (uint64_t)rbytes + 15) >> 4;
             const uint64_t line0 = ((rbase >> 7) << 3) + c * S;
             const uint64_t line1 = line0 + S < lend ? line0 + S : lend;
-            a2av_copy_short<NT>(p, d, rbase, rbytes, line0, line1, s_E, s_DW, s_meta);
+            a2av_copy_short<NT, A2avGroup>(p, d, rbase, rbytes, line0, line1, s_E, s_DW, s_meta);
         }
     }
 }

@@ -17,9 +17,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
 typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
 
-// Global-address-space views: the loads/stores become global_* (not flat_*) instructions.
+// Global-address-space views: the loads/stores become global_* (not flat_*) instructions.  (On the
+// host, where tests run some of this code, the sanitizers watch plain pointers only.)
+#ifdef __HIP_DEVICE_COMPILE__
 #define GPUMPI_GLOBAL __attribute__((address_space(1)))
-__device__ __forceinline__ u32x4 gload16(uint64_t a) {
+#else
+#define GPUMPI_GLOBAL
+#endif
+__host__ __device__ __forceinline__ u32x4 gload16(uint64_t a) {
     return *(const GPUMPI_GLOBAL u32x4_a1*)(uintptr_t)a;
 }
 // The same past the caches: data that nothing reads again soon.
@@ -27,7 +32,7 @@ __device__ __forceinline__ u32x4 gload16_nt(uint64_t a) {
     return __builtin_nontemporal_load((const GPUMPI_GLOBAL u32x4_a1*)(uintptr_t)a);
 }
 template <bool NT>
-__device__ __forceinline__ void gstore16(uint64_t a, u32x4 v) {
+__host__ __device__ __forceinline__ void gstore16(uint64_t a, u32x4 v) {
     GPUMPI_GLOBAL u32x4* p = (GPUMPI_GLOBAL u32x4*)(uintptr_t)a;
     if constexpr (NT) __builtin_nontemporal_store(v, p);
     else *p = v;

@@ -1,12 +1,19 @@
-"""CPU model of the short rows' copy (runtime/batched.h, a2av_copy_short, a2av_assemble_line
-and a2av_row_end): the window of segments, the lane's bisection, the two-segment funnel and
-the piecewise assembly are replayed over random layouts, and every row byte must be written
-once with the value that the plain definition of the exchange gives, reading no byte outside
-its segment.  The long rows' ends go through the same assembly."""
+"""The short rows' copy (runtime/batched.h: a2av_copy_short, a2av_assemble_line, a2av_row_end) on the
+CPU.  test_kernel_code runs the kernels' own code over random layouts, whole-row windows of up
+to 64 ranks and the long rows' ends among them.  test_short_row_lines is a model of the design
+alone: the window of segments found by a search (as with more than 64 ranks), the lane's
+bisection, the two-segment funnel and the piecewise assembly are restated and every row byte
+must be written once, reading no byte outside its segment."""
 import numpy as np
 import pytest
 
+from host_build import run_check
+
 WINDOW = 512
+
+
+def test_kernel_code(tmp_path):
+    run_check("a2av_short_check", tmp_path, sanitize=True)
 
 
 def assemble(rbase, rbytes, line, at, read):
