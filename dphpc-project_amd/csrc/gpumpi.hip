@@ -1368,7 +1368,8 @@ struct gpumpi_p2p_plan {
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
 };
 
-// The step's two kernels on stream s (no allocation, no host synchronisation: capturable).
+// The step's kernel on stream s, or two past kP2pFused pairs (no allocation, no host
+// synchronisation: capturable).
 static int p2p_launch(gpumpi_p2p_plan* pl, const P2pPair* pairs, int64_t n, hipStream_t s, bool timed) {
     if (timed) hipEventRecord(pl->ev[0], s);
     uint64_t* tile_chunks = pl->chunk_off + pl->max_pairs;
@@ -1382,7 +1383,8 @@ static int p2p_launch(gpumpi_p2p_plan* pl, const P2pPair* pairs, int64_t n, hipS
     // short lists: many small workgroups, each with a scan of its own (64 pairs of 16 MiB: 420
     // us, one workgroup of 16 waves per CU 436); longer ones: one scan per CU (3072 pairs of
     // 5 KiB: 9.8, small workgroups 14 to 36); lists with a scan kernel: what is resident at
-    // once (65536 pairs of 4 KiB: 127 us, one large workgroup per CU 138)
+    // once (65536 pairs of 4 KiB: 127 us, one large workgroup per CU 138).  Compared on one set of
+    // buffers with non-temporal stores; what the steps take now stands in batched_p2p.h.
     const unsigned cus = (unsigned)pl->cus;
     if (n <= kP2pShort)
         p2p_copy_kernel<kP2pShort, 256, 5><<<dim3(16 * cus), dim3(256), 0, s>>>(pairs, n, shift, pl->chunk_off, tile_chunks);

@@ -1,4 +1,5 @@
-// Batched MPI_Alltoallv step: three kernels replayed as one hipGraph per step.
+// Batched MPI_Alltoallv step: a plan, a scan and a copy kernel (plan and scan in one for up to 64
+// ranks; in pipelined graphs the copy plans the next step), replayed from hipGraphs.
 //
 // Semantics: gpu_mpi/mpi.cu:363-408 (block s of rank d's receive buffer <- block d of
 // rank s's send buffer, counts/displacements in elements), preceded by the Alltoall of

@@ -18,11 +18,13 @@
 //                    forward; a chunk is 8 unaligned 16-byte loads per lane, all issued before
 //                    its stores.
 // Lists of up to kP2pFused pairs need no scan kernel: every copy workgroup scans the whole list
-// into LDS.  Measured, us per step: 3072 pairs of 5 KiB 14.2 -> 9.8, 65536 pairs of 4 KiB 188 ->
-// 127 (one workgroup scanned them in 50), 1000 pairs of 256 KiB 118 -> 83 (the non-temporal
-// stores), 64 pairs of 16 MiB 442 -> 420.
+// into LDS.  Measured against a scan by one workgroup and cached loads and stores throughout, us
+// per step on three sets of buffers in turn: 3072 pairs of 5 KiB 14.6 -> 11.4, 65536 pairs of 4 KiB
+// 189 -> 141 (their scan, by events, 56 -> 8), 1000 pairs of 256 KiB 119 -> 116, 64 pairs of 16
+// MiB 440 -> 415.
 // HBM traffic = 2 x the bytes of the pairs (read once, written once) + 8 B per pair of
-// offsets (or 24 B per pair and CU, from the L2s).
+// offsets (or, without a scan kernel, 24 B per pair and workgroup from the L2s: 16 workgroups per
+// CU up to kP2pShort pairs, one up to kP2pFused).
 #pragma once
 
 #include "common.h"

@@ -147,7 +147,8 @@ static __global__ void gen_keys_kernel(uint32_t* keys, int P, int64_t n, uint64_
 }
 
 // ------------------------------------------------------------------ bucket plan
-// Each rank's keys are cut into tiles of consecutive keys, one workgroup per tile:
+// Each rank's keys are cut into tiles of consecutive keys, one or a few per workgroup
+// (bucket_plan.h):
 //   bucket_tile_hist  the tile's keys per bucket
 //   bucket_rank_scan  per rank: exclusive prefix of the tiles' counts within each bucket, and
 //                     of the buckets within the rank
@@ -155,9 +156,10 @@ static __global__ void gen_keys_kernel(uint32_t* keys, int P, int64_t n, uint64_
 //   bucket_splitters  which buckets each rank receives
 //   bucket_scatter    the tile's keys to their stable places; the first tile of a rank also
 //                     writes the rank's send counts and displacements
-// HBM traffic: the keys read twice and written once, plus 4 table passes of 4 B per tile and
-// bucket.  Measured at 512 ranks x 2^18 keys, 1024 buckets: tile_hist 145 us (3.7 TB/s read; the
-// LDS atomics bound it, 256 threads per workgroup took 158), rank_scan 17, colsum 11, splitters 5, scatter 328 us (3.3 TB/s).  One wavefront per rank, 64
+// HBM traffic: the keys read twice and written once, plus 4 table passes of 4 B per workgroup
+// and bucket.  Measured at 512 ranks x 2^18 keys, 1024 buckets: tile_hist 145-150 us (3.7 TB/s
+// read; the LDS atomics bound it, 256 threads per workgroup took 158), rank_scan 16, colsum 11,
+// splitters 5, scatter 321 us (3.3 TB/s).  One wavefront per rank, 64
 // keys per step (the former scatter), was a serial chain of n / 64 steps on P waves: 5676 us
 // there and 208 us at 4 ranks x 2^14, now 8.5; the column sums by one thread per bucket 139 us.
 constexpr int kBucketThreads = 1024;
