@@ -2,7 +2,9 @@
 
 The copy kernel writes a row's 16-byte destination lines from several code paths: whole
 lines inside one segment, lines that straddle segments (inline dword assembly, or the
-straddle threads in deferred mode), and lines at a row's ends (byte path).  This model
+straddle threads in deferred mode), and lines at a row's ends (a lane each before the loop, or
+the loop's byte path in deferred mode).  The short rows have a loop of their own
+(test_a2av_short.py, which also runs the row ends' code itself).  This model
 replays the kernels' index arithmetic -- chunk rows and line ranges (scan), the 64-segment
 LDS window and its coverage, the wave cursor and the four-entry selection (copy), the
 owner rule of the straddle threads -- over random layouts with unaligned receive rows,
@@ -82,8 +84,26 @@ def seg_global(seg_end, seg_src, d, rbase, q):
     return st, int(se[k]), int(seg_src[d, k]) - (rbase + st)
 
 
+def row_end(seg_end, seg_src, row_bytes, recv_addr, d, which, mem):
+    """a2av_row_end: the row's first or last line, if it holds bytes of the row and others."""
+    rbase, rbytes = recv_addr[d], int(row_bytes[d])
+    rend = rbase + rbytes
+    if rbytes == 0 or (rend if which else rbase) % 16 == 0:
+        return
+    first, last = rbase >> 4, rend >> 4
+    if which and first == last and rbase % 16:
+        return
+    line = last if which else first
+    for a in range(max(line << 4, rbase), min((line + 1) << 4, rend)):
+        st, en, D = seg_global(seg_end, seg_src, d, rbase, a - rbase)
+        mem.write(a, mem.src(a + D), d)
+
+
 def copy_kernel(P, seg_end, seg_src, row_bytes, recv_addr, chunk_off, C, U, defer, mem):
     """a2av_copy_kernel<U, NT, defer> over every chunk."""
+    if not defer:
+        for g in range(2 * P):
+            row_end(seg_end, seg_src, row_bytes, recv_addr, g >> 1, g & 1, mem)
     for ch in range(int(chunk_off[P])):
         d = search_le(chunk_off, P, ch)
         c = ch - int(chunk_off[d])
@@ -134,7 +154,7 @@ def copy_kernel(P, seg_end, seg_src, row_bytes, recv_addr, chunk_off, C, U, defe
             def boundary(line):  # a2av_boundary_line<defer>
                 la = line << 4
                 off = la - rbase
-                if defer and off >= 0 and off + 16 <= rbytes:
+                if defer == (off >= 0 and off + 16 <= rbytes):
                     return
                 for i in range(4):
                     q = off + 4 * i

@@ -1,6 +1,7 @@
 """CPU replay of the batched point-to-point step's work split (runtime/batched_p2p.h): the
 scan's chunk offsets, each wave's equal range of chunks, the 64-ary search for the wave's
-first pair, the forward walk over empty pairs, and each chunk's piece of its destination.
+first pair (of a list that the copy's workgroups scan; longer ones search their tiles first, which
+test_gpu_p2p_lists.py covers), the forward walk over empty pairs, and each chunk's piece of its destination.
 Over random pair lists and wave counts, every destination byte of every pair is written
 exactly once and no byte outside the pairs is written; every piece's aligned interior fits
 one chunk (at most 8 vectors per lane) with heads and tails under 16 bytes."""
